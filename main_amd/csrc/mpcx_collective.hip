@@ -286,21 +286,6 @@ struct Dimer {
   double v[12][2 * ND];
 };
 
-template <int ND>
-__device__ __forceinline__ void dimer_load(Dimer<ND>& d, const double (*sd)[MAXS]) {
-#pragma unroll
-  for (int f = 0; f < 12; f++)
-#pragma unroll
-    for (int s = 0; s < 2 * ND; s++) d.v[f][s] = sd[f][s];
-}
-template <int ND>
-__device__ __forceinline__ void dimer_store(const Dimer<ND>& d, double (*sd)[MAXS]) {
-#pragma unroll
-  for (int f = 0; f < 12; f++)
-#pragma unroll
-    for (int s = 0; s < 2 * ND; s++) sd[f][s] = d.v[f][s];
-}
-
 // evolve_mod.f95:325-415: Q = V + h F, advance, RATTLE on the bond length.
 template <int ND>
 __device__ __forceinline__ void rattle_positions(const CoP& P, Dimer<ND>& d, int* err) {
@@ -372,110 +357,47 @@ __device__ __forceinline__ void lj_mot_mot(const CoP& P, double x1, double y1, d
   }
 }
 
-// forces_mod.f95:303-333 with the dummy order of the call at evolve_mod.f95:597-600
+// forces_mod.f95:303-333 with the dummy order of the call at evolve_mod.f95:
+// 597-600: force and potential of the upper wall, then the lower one added.
+// The terms are a call: a sphere is seldom within a wall's cutoff, and the
+// inlined pow (four copies in a dimer's step) spilled the step's registers.
+struct WallTerm { double f, pot; };
+__device__ __attribute__((noinline)) WallTerm lj_wall_term(double dR, double pe, double R3, double R9, double r9R9,
+                                                           double r3R3) {
+  const double IdRsq = 1.0 / (dR * dR);
+  const double IdR3 = pow(IdRsq, 1.5);
+  const double IdR9 = (IdR3 * IdR3) * IdR3;
+  const double IdR5 = IdR3 * IdRsq;
+  const double IdR11 = IdR9 * IdRsq;
+  return WallTerm{(pe * (r9R9 * IdR11 - r3R3 * IdR5)) * dR, pe * (R9 * IdR9 - R3 * IdR3)};
+}
 __device__ __forceinline__ void lj_mot_wall(const CoP& P, double zd, int i, double& fw, double& pot) {
-  const double R3 = P.wR3[i], R9 = P.wR9[i], r9R9 = P.wA[i], r3R3 = P.wB[i];
-  const double pe = P.pref * P.Ew;
   fw = 0.0;
   pot = 0.0;
-  double dR = P.box[2] - zd;
-  if (dR * dR < P.wcut2[i]) {
-    double IdRsq = 1.0 / (dR * dR);
-    double IdR3 = pow(IdRsq, 1.5);
-    double IdR9 = (IdR3 * IdR3) * IdR3;
-    double IdR5 = IdR3 * IdRsq;
-    double IdR11 = IdR9 * IdRsq;
-    fw = (pe * (r9R9 * IdR11 - r3R3 * IdR5)) * dR;
-    pot = pe * (R9 * IdR9 - R3 * IdR3) + 1.0;
+  const double up = P.box[2] - zd, lo = 0.0 - zd;
+  const double c2 = P.wcut2[i];
+  if (!(up * up < c2 || lo * lo < c2)) return;
+  const double pe = P.pref * P.Ew;
+  if (up * up < c2) {
+    const WallTerm t = lj_wall_term(up, pe, P.wR3[i], P.wR9[i], P.wA[i], P.wB[i]);
+    fw = t.f;
+    pot = t.pot + 1.0;
   }
-  dR = 0.0 - zd;
-  if (dR * dR < P.wcut2[i]) {
-    double IdRsq = 1.0 / (dR * dR);
-    double IdR3 = pow(IdRsq, 1.5);
-    double IdR9 = (IdR3 * IdR3) * IdR3;
-    double IdR5 = IdR3 * IdRsq;
-    double IdR11 = IdR9 * IdRsq;
-    fw = fw + (pe * (r9R9 * IdR11 - r3R3 * IdR5)) * dR;
-    pot = (pot + pe * (R9 * IdR9 - R3 * IdR3)) + 1.0;
+  if (lo * lo < c2) {
+    const WallTerm t = lj_wall_term(lo, pe, P.wR3[i], P.wR9[i], P.wA[i], P.wB[i]);
+    fw = fw + t.f;
+    pot = (pot + t.pot) + 1.0;
   }
 }
 
-// evolve_mod.f95:605-636 (solvent sums arrive as tree-reduced totals) and
-// :679-724 (velocity RATTLE).  sumF[4*s + 0..2] = sum of Fpair of sphere s,
-// sumF[4*s + 3] = sum of its Potential.
-template <int ND>
-__device__ __forceinline__ void dimer_forces_and_rattle_v(const CoP& P, Dimer<ND>& d, const double* sumF,
-                                                          double& tpot, int* err) {
-  double tpp[2 * ND];
-#pragma unroll
-  for (int k = 0; k < ND; k++)
-#pragma unroll
-    for (int i = 0; i < 2; i++) {
-      const int s = k + i * ND;
-      double fw, wp;
-      lj_mot_wall(P, d.v[DZ][s], i, fw, wp);
-      double fx = 0.0 - sumF[4 * s + 0], fy = 0.0 - sumF[4 * s + 1], fz = 0.0 - sumF[4 * s + 2];
-      double tp = 0.0 + sumF[4 * s + 3];
-#pragma unroll
-      for (int j = 0; j < ND; j++)
-#pragma unroll
-        for (int l = 0; l < 2; l++) {
-          if (j == k) continue;   // Fmot(k,i,k,l) stays zero (evolve_mod.f95:580)
-          const int b = j + l * ND;
-          const int kind = (i == 0 && l == 0) ? 0 : (i == 1 && l == 1) ? 2 : 1;
-          double mx, my, mz, mp;
-          lj_mot_mot(P, d.v[DX][s], d.v[DY][s], d.v[DZ][s], d.v[DX][b], d.v[DY][b], d.v[DZ][b], kind, mx, my, mz,
-                     mp);
-          fx = fx + mx; fy = fy + my; fz = fz + mz;
-          if (j < k) tp = tp + mp;
-        }
-      fz = fz + fw;
-      tp = tp + wp;
-      d.v[DFX][s] = fx; d.v[DFY][s] = fy; d.v[DFZ][s] = fz;
-      tpp[s] = tp;
-    }
-  tpot = 0.0;
-#pragma unroll
-  for (int k = 0; k < ND; k++)
-#pragma unroll
-    for (int i = 0; i < 2; i++) tpot = tpot + tpp[k + i * ND];
-#pragma unroll
-  for (int k = 0; k < ND; k++) {
-    const int s0 = k, s1 = k + ND;
-    d.v[DVX][s0] = d.v[DQX][s0] + P.hc * d.v[DFX][s0];
-    d.v[DVY][s0] = d.v[DQY][s0] + P.hc * d.v[DFY][s0];
-    d.v[DVZ][s0] = d.v[DQZ][s0] + P.hc * d.v[DFZ][s0];
-    d.v[DVX][s1] = d.v[DQX][s1] + P.hn * d.v[DFX][s1];
-    d.v[DVY][s1] = d.v[DQY][s1] + P.hn * d.v[DFY][s1];
-    d.v[DVZ][s1] = d.v[DQZ][s1] + P.hn * d.v[DFZ][s1];
-    for (long long acc = 0;; acc++) {
-      if (acc == RATTLE_CAP) { raise_error(err, ERR_RATTLE); break; }
-      double dvx = d.v[DVX][s0] - d.v[DVX][s1], dvy = d.v[DVY][s0] - d.v[DVY][s1], dvz = d.v[DVZ][s0] - d.v[DVZ][s1];
-      double d0 = pbc_half(d.v[DX][s0] - d.v[DX][s1], P.box[0]);
-      double d1 = pbc_half(d.v[DY][s0] - d.v[DY][s1], P.box[1]);
-      double d2 = d.v[DZ][s0] - d.v[DZ][s1];
-      double c2 = 2.0 * (dvx * d0 + dvy * d1 + dvz * d2);
-      if (fabs(c2) < 1e-8) break;
-      double O = -((0.25 * (P.IIMcIMn * c2)) / P.Dcn2);
-      double o2 = 2.0 * O;
-      d.v[DVX][s0] = d.v[DVX][s0] + (o2 * d0) / P.Mc;
-      d.v[DVY][s0] = d.v[DVY][s0] + (o2 * d1) / P.Mc;
-      d.v[DVZ][s0] = d.v[DVZ][s0] + (o2 * d2) / P.Mc;
-      d.v[DVX][s1] = d.v[DVX][s1] - (o2 * d0) / P.Mn;
-      d.v[DVY][s1] = d.v[DVY][s1] - (o2 * d1) / P.Mn;
-      d.v[DVZ][s1] = d.v[DVZ][s1] - (o2 * d2) / P.Mn;
-    }
-  }
-}
-
-// Wave forms of the one-dimer step: every lane of the wave holds the dimer
+// Wave forms of one dimer's step: every lane of the wave holds the dimer
 // and computes the same scalars; in each RATTLE iteration lane c (0..5)
 // updates component c of the update -- sphere c / 3, axis c % 3 -- with the
-// expression of the one-thread form above, and the six results are read back
-// from lanes 0..5 into every lane.  The results are bitwise those of the
-// one-thread form, and an iteration's chain holds two or three divisions
-// instead of twelve (a wave issues every instruction whatever lanes are
-// active).  Lane 0 alone reports errors.
+// expression of the one-thread form (rattle_positions above, ge_rattle_v), and
+// the six results are read back from lanes 0..5 into every lane.  The results
+// are bitwise those of the one-thread form, and an iteration's chain holds two
+// or three divisions instead of twelve (a wave issues every instruction
+// whatever lanes are active).  Lane 0 alone reports errors.
 __device__ __forceinline__ double pick6(int c, double a0, double a1, double a2, double b0, double b1, double b2) {
   return c < 3 ? (c == 0 ? a0 : c == 1 ? a1 : a2) : (c == 3 ? b0 : c == 4 ? b1 : b2);
 }
@@ -530,23 +452,44 @@ __device__ __forceinline__ void rattle_positions_wave(const CoP& P, Dimer<1>& d,
   }
   bcast6(q, d.v[DQX][0], d.v[DQY][0], d.v[DQZ][0], d.v[DQX][1], d.v[DQY][1], d.v[DQZ][1]);
 }
+// evolve_mod.f95:605-636 (solvent sums arrive as tree-reduced totals) and
+// :679-724 (velocity RATTLE) of dimer k of ND.  sumF[4*i + 0..2] = sum of Fpair
+// of its sphere i, sumF[4*i + 3] = sum of its Potential; pos holds the
+// positions of every sphere of the system at this step.
+template <int ND>
 __device__ __forceinline__ void dimer_forces_and_rattle_v_wave(const CoP& P, Dimer<1>& d, const double* sumF,
-                                                               double& tpot, int* err, int lane) {
-  double tpp[2];
+                                                               const double (*pos)[MAXS], int k, double (&tpp)[2],
+                                                               int* err, int lane) {
+  // sphere-sphere terms (none with one dimer: Fmot(k,i,k,l) stays zero,
+  // evolve_mod.f95:580): lane i*NP + q for sphere i and the q-th sphere of the
+  // other dimers, read back in the reference's order
+  constexpr int NP = 2 * (ND - 1);
+  double mx = 0.0, my = 0.0, mz = 0.0, mp = 0.0;
+  if (ND > 1 && lane < 2 * NP) {
+    const int i = lane / (NP > 0 ? NP : 1), q = lane % (NP > 0 ? NP : 1);
+    const int j = (q >> 1) + ((q >> 1) >= k ? 1 : 0), l = q & 1, b = j + l * ND;
+    const int kind = (i == 0 && l == 0) ? 0 : (i == 1 && l == 1) ? 2 : 1;
+    lj_mot_mot(P, i ? d.v[DX][1] : d.v[DX][0], i ? d.v[DY][1] : d.v[DY][0], i ? d.v[DZ][1] : d.v[DZ][0], pos[DX][b],
+               pos[DY][b], pos[DZ][b], kind, mx, my, mz, mp);
+  }
 #pragma unroll
-  for (int i = 0; i < 2; i++) {   // one dimer: no sphere-sphere terms (evolve_mod.f95:580)
+  for (int i = 0; i < 2; i++) {
     double fw, wp;
     lj_mot_wall(P, d.v[DZ][i], i, fw, wp);
     double fx = 0.0 - sumF[4 * i + 0], fy = 0.0 - sumF[4 * i + 1], fz = 0.0 - sumF[4 * i + 2];
     double tp = 0.0 + sumF[4 * i + 3];
+#pragma unroll
+    for (int q = 0; q < NP; q++) {
+      fx = fx + lane_read_d(mx, i * NP + q);
+      fy = fy + lane_read_d(my, i * NP + q);
+      fz = fz + lane_read_d(mz, i * NP + q);
+      if ((q >> 1) < k) tp = tp + lane_read_d(mp, i * NP + q);
+    }
     fz = fz + fw;
     tp = tp + wp;
     d.v[DFX][i] = fx; d.v[DFY][i] = fy; d.v[DFZ][i] = fz;
     tpp[i] = tp;
   }
-  tpot = 0.0;
-  tpot = tpot + tpp[0];
-  tpot = tpot + tpp[1];
   d.v[DVX][0] = d.v[DQX][0] + P.hc * d.v[DFX][0];
   d.v[DVY][0] = d.v[DQY][0] + P.hc * d.v[DFY][0];
   d.v[DVZ][0] = d.v[DQZ][0] + P.hc * d.v[DFZ][0];

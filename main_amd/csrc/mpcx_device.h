@@ -111,6 +111,16 @@ __device__ __forceinline__ double lane_read_d(double v, int lane) {
   return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
 }
 constexpr int DPP_QUAD_1032 = 0xb1, DPP_QUAD_2301 = 0x4e, DPP_ROW_MIRROR = 0x140, DPP_ROW_HALF_MIRROR = 0x141;
+constexpr int DPP_ROW_SHL4 = 0x104, DPP_ROW_SHR4 = 0x114, DPP_ROW_ROR8 = 0x128;
+// v of lane ^ 4: quads 0 and 2 of a row take it from four lanes up, 1 and 3 from four down
+__device__ __forceinline__ double dpp_xor4_d(double v) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  int lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)b, DPP_ROW_SHL4, 0xf, 0x5, false);
+  int hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(b >> 32), DPP_ROW_SHL4, 0xf, 0x5, false);
+  lo = __builtin_amdgcn_update_dpp(lo, (int)(unsigned)b, DPP_ROW_SHR4, 0xf, 0xa, false);
+  hi = __builtin_amdgcn_update_dpp(hi, (int)(unsigned)(b >> 32), DPP_ROW_SHR4, 0xf, 0xa, false);
+  return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
+}
 __device__ __forceinline__ double wave_sum_dpp(double v) {
   v = v + dpp_mov_d<DPP_QUAD_1032>(v);
   v = v + dpp_mov_d<DPP_QUAD_2301>(v);
