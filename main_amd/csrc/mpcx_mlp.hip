@@ -19,148 +19,311 @@ namespace mpcx {
 namespace ml {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int GT = 256;                 // GEMM block: 4 waves
-constexpr int BM = 64, BN = 64, BK = 32;
+// ------------------------------------------------------------------ layouts
+// Every product is C[m][n] = sum_k A[m][k] B[n][k] of two BF16 operands whose
+// contraction index is contiguous, so a lane's fragment of eight is one 16-byte
+// load from L2 and no operand is staged, transposed or bounds-checked on the
+// way: the weights are kept as W (n_next x n_prev) and as its transpose, and a
+// layer's activations and gradients are written by the product that makes them
+// both by row and transposed, with zeros up to the next multiple of 32.
+// (Element-wise staging through LDS with a 64 x 64 block tile left 4 to 33
+// workgroups a product and 22 us of loads in each: a training step of the
+// 8-256-256-256-2049 network, batch 64, took 460 us.)
+constexpr int PAD = 32;
+static inline int up32(int n) { return (n + PAD - 1) / PAD * PAD; }
 
 __device__ __forceinline__ __bf16 to_bf16(float f) { return (__bf16)f; }   // round to nearest even
 
-// C[m][n] (ldc) = act(sum_k A[m*am + k*ak] * B[k*bk + n*bn] + bias[n]) (+ C if accumulate);
-// A, B in BF16, accumulation in FP32.  Each wave owns a 32x32 quarter of the
-// 64x64 block tile: 2x2 MFMA 16x16x32 tiles.  Z (optional) keeps the
-// pre-activation for the backward pass.
-__global__ __launch_bounds__(GT) void gemm_bf16(int M, int N, int K, const __bf16* __restrict__ A, long long am,
-                                                long long ak, const __bf16* __restrict__ B, long long bk, long long bn,
-                                                float* __restrict__ C, long long ldc, const float* __restrict__ bias,
-                                                int relu, float* __restrict__ Z, __bf16* __restrict__ Cb,
-                                                int accumulate) {
-  __shared__ __bf16 As[BM][BK + 8];   // +8: 16-byte row padding against LDS bank conflicts
-  __shared__ __bf16 Bs[BN][BK + 8];   // B tile stored transposed: Bs[n][k]
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-  const int wm = (w >> 1) * 32, wn = (w & 1) * 32;
-  f32x4 acc[2][2];
+// One wave's tile of 16 TM x 16 TN.  Loads run U steps of 32 ahead of the
+// matrix instructions (65 steps at the widest contraction, one wave a SIMD:
+// latency, not rate, bounds the small products).  Accumulation over k is in
+// ascending order whatever the tile.
+template <int TM, int TN>
+__device__ __forceinline__ void tile_product(const __bf16* __restrict__ A, int lda, const __bf16* __restrict__ B, int ldb,
+                                             int K, int m0, int n0, f32x4 (&acc)[TM][TN]) {
+  constexpr int U = TM * TN > 1 ? 2 : 4;
+  const int lane = threadIdx.x & 63, rr = lane & 15, kq = (lane >> 4) * 8;
+  const __bf16* pa = A + (size_t)(m0 + rr) * lda + kq;
+  const __bf16* pb = B + (size_t)(n0 + rr) * ldb + kq;
 #pragma unroll
-  for (int i = 0; i < 2; i++)
+  for (int i = 0; i < TM; i++)
 #pragma unroll
-    for (int j = 0; j < 2; j++) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
-  for (int k0 = 0; k0 < K; k0 += BK) {
-    // stage the tiles (zero beyond the matrix edges): 64x32 elements each, 8 per thread
-    for (int e = tid; e < BM * BK; e += GT) {
-      const int r = e / BK, c = e % BK;
-      const int gm = m0 + r, gk = k0 + c;
-      As[r][c] = (gm < M && gk < K) ? A[gm * am + gk * ak] : to_bf16(0.f);
-      const int gn = n0 + r;
-      Bs[r][c] = (gn < N && gk < K) ? B[gk * bk + gn * bn] : to_bf16(0.f);
-    }
-    __syncthreads();
-    // fragments: lane l holds row/column l%16 and k = 8*(l/16) .. +7
-    const int rr = lane & 15, kq = (lane >> 4) * 8;
-    bf16x8 a[2], b[2];
+    for (int j = 0; j < TN; j++) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  bf16x8 a[U][TM], b[U][TN];
+  auto fetch = [&](int k0) {
 #pragma unroll
-    for (int i = 0; i < 2; i++) {
+    for (int u = 0; u < U; u++)
+      if (k0 + u * 32 < K) {
 #pragma unroll
-      for (int t = 0; t < 8; t++) {
-        a[i][t] = As[wm + i * 16 + rr][kq + t];
-        b[i][t] = Bs[wn + i * 16 + rr][kq + t];
+        for (int i = 0; i < TM; i++) a[u][i] = *(const bf16x8*)(pa + (size_t)i * 16 * lda + k0 + u * 32);
+#pragma unroll
+        for (int j = 0; j < TN; j++) b[u][j] = *(const bf16x8*)(pb + (size_t)j * 16 * ldb + k0 + u * 32);
       }
+  };
+  fetch(0);
+  for (int k0 = 0; k0 < K; k0 += U * 32) {
+    bf16x8 ca[U][TM], cb[U][TN];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+#pragma unroll
+      for (int i = 0; i < TM; i++) ca[u][i] = a[u][i];
+#pragma unroll
+      for (int j = 0; j < TN; j++) cb[u][j] = b[u][j];
     }
+    if (k0 + U * 32 < K) fetch(k0 + U * 32);
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+    for (int u = 0; u < U; u++)
+      if (k0 + u * 32 < K) {
 #pragma unroll
-      for (int j = 0; j < 2; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
-    __syncthreads();
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+          for (int j = 0; j < TN; j++)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ca[u][i], cb[u][j], acc[i][j], 0, 0, 0);
+      }
   }
-  // result of tile (i,j): lane l holds column l%16, rows 4*(l/16) .. +3
-  const int cc = lane & 15, rq = (lane >> 4) * 4;
+}
+// the wave's tile of a grid of mt x nt tiles, four waves a workgroup along n
+// (then along m): first output row and column, or false beyond the last
+template <int TM, int TN>
+__device__ __forceinline__ bool my_tile(int mt, int nt, int blk, int& m0, int& n0) {
+  const int t = blk * 4 + (threadIdx.x >> 6);
+  if (t >= mt * nt) return false;
+  m0 = (t / nt) * 16 * TM;
+  n0 = (t % nt) * 16 * TN;
+  return true;
+}
+// element (i, j, t) of a lane: column lane % 16, rows 4 (lane / 16) + t
+#define TILE_ROW(i) (m0 + (i)*16 + ((int)(threadIdx.x & 63) >> 4) * 4)
+#define TILE_COL(j) (n0 + (j)*16 + (int)(threadIdx.x & 15))
+
+__device__ __forceinline__ void store4(__bf16* p, const float (&v)[4]) {   // four consecutive, 8-byte aligned
+  bf16x4 o;
 #pragma unroll
-  for (int i = 0; i < 2; i++)
+  for (int t = 0; t < 4; t++) o[t] = to_bf16(v[t]);
+  *(bf16x4*)p = o;
+}
+
+// A layer's activations or gradients: FP32 by row (may be null), BF16 by row
+// and transposed (null where nothing reads them)
+struct Act {
+  float* f;
+  __bf16* b;
+  __bf16* t;
+  int cols, ldb, ldt;
+};
+
+// H = act(A W^T + bias), rows < rows; the rows up to the next multiple of 32
+// are written as zeros (dW's contraction runs over them).
+template <int TM, int TN>
+__global__ __launch_bounds__(256) void layer_forward(int rows, int mt, int nt, int K, const __bf16* __restrict__ A, int lda,
+                                                     const __bf16* __restrict__ W, int ldw,
+                                                     const float* __restrict__ bias, int relu, Act H) {
+  int m0, n0;
+  if (!my_tile<TM, TN>(mt, nt, blockIdx.x, m0, n0)) return;
+  f32x4 acc[TM][TN];
+  tile_product<TM, TN>(A, lda, W, ldw, K, m0, n0, acc);
 #pragma unroll
-    for (int j = 0; j < 2; j++)
+  for (int j = 0; j < TN; j++) {
+    const int gn = TILE_COL(j);
+    if (gn >= H.cols) continue;
+    const float bv = bias ? bias[gn] : 0.f;
+#pragma unroll
+    for (int i = 0; i < TM; i++) {
+      const int gm = TILE_ROW(i);
+      float v[4];
 #pragma unroll
       for (int t = 0; t < 4; t++) {
-        const int gm = m0 + wm + i * 16 + rq + t, gn = n0 + wn + j * 16 + cc;
-        if (gm >= M || gn >= N) continue;
-        float v = acc[i][j][t];
-        if (bias) v = v + bias[gn];
-        if (Z) Z[gm * ldc + gn] = v;
-        if (relu) v = v > 0.f ? v : 0.f;
-        if (accumulate) v = v + C[gm * ldc + gn];
-        C[gm * ldc + gn] = v;
-        if (Cb) Cb[gm * ldc + gn] = to_bf16(v);
+        v[t] = acc[i][j][t] + bv;
+        if (relu) v[t] = v[t] > 0.f ? v[t] : 0.f;
+        if (gm + t >= rows) v[t] = 0.f;
+        if (H.f && gm + t < rows) H.f[(size_t)(gm + t) * H.cols + gn] = v[t];
+        if (H.b) H.b[(size_t)(gm + t) * H.ldb + gn] = to_bf16(v[t]);
       }
+      if (H.t) store4(H.t + (size_t)gn * H.ldt + gm, v);
+    }
+  }
 }
 
-__global__ void to_bf16_kernel(const float* __restrict__ x, __bf16* __restrict__ y, long long n) {
-  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
-    y[i] = to_bf16(x[i]);
+// The output layer of a training step with its loss: Y = A W^T + bias stays in
+// registers; the wave's share of sum_c wout[c] (Y - T)^2 goes to part[tile],
+// the gradient 2 w (Y - T) / rows to dZ.  Target row r is row idx[r] of T
+// (idx null: row r).
+__global__ __launch_bounds__(256) void output_loss(int rows, int mt, int nt, int K, const __bf16* __restrict__ A, int lda,
+                                                   const __bf16* __restrict__ W, int ldw, const float* __restrict__ bias,
+                                                   const float* __restrict__ T, const int* __restrict__ idx,
+                                                   const float* __restrict__ wout, Act dZ, double* __restrict__ part) {
+  int m0, n0;
+  if (!my_tile<1, 1>(mt, nt, blockIdx.x, m0, n0)) return;
+  const int gn = TILE_COL(0), gm = TILE_ROW(0);
+  const bool col = gn < dZ.cols;
+  float tv[4];   // the targets' loads run beside the product
+#pragma unroll
+  for (int t = 0; t < 4; t++)
+    tv[t] = col && gm + t < rows ? T[(size_t)(idx ? idx[gm + t] : gm + t) * dZ.cols + gn] : 0.f;
+  const float bv = col ? bias[gn] : 0.f, wv = col ? wout[gn] : 0.f;
+  f32x4 acc[1][1];
+  tile_product<1, 1>(A, lda, W, ldw, K, m0, n0, acc);
+  double loss = 0.0;
+  float g[4];
+#pragma unroll
+  for (int t = 0; t < 4; t++) {
+    g[t] = 0.f;
+    if (!col || gm + t >= rows) continue;
+    const float d = (acc[0][0][t] + bv) - tv[t];
+    loss += (double)wv * (double)d * (double)d;
+    g[t] = 2.f * wv * d / (float)rows;
+    dZ.f[(size_t)(gm + t) * dZ.cols + gn] = g[t];
+  }
+  if (col) {
+#pragma unroll
+    for (int t = 0; t < 4; t++) dZ.b[(size_t)(gm + t) * dZ.ldb + gn] = to_bf16(g[t]);
+    store4(dZ.t + (size_t)gn * dZ.ldt + gm, g);
+  }
+  loss = wave_sum(loss);
+  if ((threadIdx.x & 63) == 0) part[blockIdx.x * 4 + (threadIdx.x >> 6)] = loss;
+}
+// loss of each step of an epoch: its tiles' shares in tile order (one wave a step)
+__global__ __launch_bounds__(64) void loss_sums(int tiles, long long stride, const double* __restrict__ part,
+                                                double* __restrict__ loss) {
+  double s = 0.0;
+  for (int j = threadIdx.x; j < tiles; j += 64) s += part[blockIdx.x * stride + j];
+  s = wave_sum(s);
+  if (threadIdx.x == 0) loss[blockIdx.x] = s;
 }
 
-// rows of x gathered by idx (a minibatch), in FP32 and BF16
-__global__ void gather_rows(const float* __restrict__ src, const int* __restrict__ idx, int rows, int cols,
-                            float* __restrict__ dst, __bf16* __restrict__ dstb) {
+// dZ_l = (dZ_{l+1} W) * (H_l > 0), A = dZ_{l+1} by row, WT the transposed weights
+__global__ __launch_bounds__(256) void layer_backward(int rows, int mt, int nt, int K, const __bf16* __restrict__ A, int lda,
+                                                      const __bf16* __restrict__ WT, int ldw, const float* __restrict__ H,
+                                                      Act dZ) {
+  int m0, n0;
+  if (!my_tile<1, 1>(mt, nt, blockIdx.x, m0, n0)) return;
+  const int gn = TILE_COL(0), gm = TILE_ROW(0);
+  const bool col = gn < dZ.cols;
+  bool on[4];
+#pragma unroll
+  for (int t = 0; t < 4; t++) on[t] = col && gm + t < rows && H[(size_t)(gm + t) * dZ.cols + gn] > 0.f;
+  f32x4 acc[1][1];
+  tile_product<1, 1>(A, lda, WT, ldw, K, m0, n0, acc);
+  if (!col) return;
+  float g[4];
+#pragma unroll
+  for (int t = 0; t < 4; t++) {
+    g[t] = on[t] ? acc[0][0][t] : 0.f;
+    if (gm + t < rows) dZ.f[(size_t)(gm + t) * dZ.cols + gn] = g[t];
+    dZ.b[(size_t)(gm + t) * dZ.ldb + gn] = to_bf16(g[t]);
+  }
+  store4(dZ.t + (size_t)gn * dZ.ldt + gm, g);
+}
+
+// Adam on one FP32 master parameter
+struct Adam {
+  float lr, b1, b2, eps, c1, c2;
+  int on;
+};
+__device__ __forceinline__ float adam_one(const Adam& a, float p, float gi, float* __restrict__ m, float* __restrict__ v) {
+  const float mi = a.b1 * *m + (1.f - a.b1) * gi;
+  const float vi = a.b2 * *v + (1.f - a.b2) * gi * gi;
+  *m = mi;
+  *v = vi;
+  return p - a.lr * (mi / a.c1) / (sqrtf(vi / a.c2) + a.eps);
+}
+
+// Weight and bias gradients of up to MAXL layers in one launch, and the Adam
+// step on them where they are made (a.on; else the gradients go to g): dW_l =
+// dZ_{l+1}^T H_l over the batch, db_l the column sums of dZ_{l+1} in row order.
+// Nothing else of the step reads the weights any more, so the BF16 copies are
+// renewed here too.
+constexpr int MAXL = 8;
+struct GradLayer {
+  const __bf16 *dZt, *Ht;   // transposed, contraction over the batch
+  const float* dZ;          // FP32 by row, for the bias
+  __bf16 *w, *wt;           // BF16 copies of the weights
+  long long woff, boff;     // in the flat parameters
+  int N, K, ldw, ldwt, nt;  // dims, leading dimensions, tiles along K
+  int blk0, bias0;          // first workgroup of its tiles and of its bias
+};
+struct GradArgs {
+  GradLayer l[MAXL];
+  int n;
+};
+__global__ __launch_bounds__(256) void layer_grads(GradArgs G, int rows, int ldt, Adam a, float* __restrict__ p,
+                                                   float* __restrict__ g, float* __restrict__ m, float* __restrict__ v) {
+  int q = 0;
+  while (q + 1 < G.n && (int)blockIdx.x >= G.l[q + 1].blk0) q++;
+  const GradLayer& L = G.l[q];
+  if ((int)blockIdx.x >= L.bias0) {
+    const int c = ((int)blockIdx.x - L.bias0) * 256 + (int)threadIdx.x;
+    if (c >= L.N) return;
+    float s = 0.f;
+    for (int r0 = 0; r0 < rows; r0 += 16) {   // sixteen loads in flight, added in row order
+      float x[16];
+#pragma unroll
+      for (int r = 0; r < 16; r++) x[r] = r0 + r < rows ? L.dZ[(size_t)(r0 + r) * L.N + c] : 0.f;
+#pragma unroll
+      for (int r = 0; r < 16; r++)
+        if (r0 + r < rows) s += x[r];
+    }
+    const long long o = L.boff + c;
+    if (a.on) p[o] = adam_one(a, p[o], s, m + o, v + o);
+    else g[o] = s;
+    return;
+  }
+  int m0, n0;
+  if (!my_tile<1, 1>((L.N + 15) / 16, L.nt, (int)blockIdx.x - L.blk0, m0, n0)) return;
+  const int gn = TILE_COL(0), gm = TILE_ROW(0);
+  f32x4 acc[1][1];
+  tile_product<1, 1>(L.dZt, ldt, L.Ht, ldt, (rows + PAD - 1) / PAD * PAD, m0, n0, acc);
+  if (gn >= L.K) return;
+  float w[4];
+#pragma unroll
+  for (int t = 0; t < 4; t++) {
+    w[t] = 0.f;
+    if (gm + t >= L.N) continue;
+    const long long o = L.woff + (long long)(gm + t) * L.K + gn;
+    if (!a.on) { g[o] = acc[0][0][t]; continue; }
+    w[t] = adam_one(a, p[o], acc[0][0][t], m + o, v + o);
+    p[o] = w[t];
+    L.w[(size_t)(gm + t) * L.ldw + gn] = to_bf16(w[t]);
+  }
+  if (a.on) store4(L.wt + (size_t)gn * L.ldwt + gm, w);
+}
+
+// BF16 copies of one layer's weights, by row and transposed
+__global__ void weights_bf16(int N, int K, const float* __restrict__ W, __bf16* __restrict__ w, int ldw,
+                             __bf16* __restrict__ wt, int ldwt) {
+  for (long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x; e < (long long)N * K;
+       e += (long long)gridDim.x * blockDim.x) {
+    const int n = (int)(e / K), k = (int)(e % K);
+    const __bf16 b = to_bf16(W[e]);
+    w[(size_t)n * ldw + k] = b;
+    wt[(size_t)k * ldwt + n] = b;
+  }
+}
+
+// The input rows of every batch of an epoch, BF16 by row and transposed, zeros
+// to the batches' padded sizes: row r of batch s is row idx[s*batch + r] of X
+// (idx null: row s*batch + r).
+__global__ void input_rows(int n, int batch, int steps, int cols, const float* __restrict__ X, const int* __restrict__ idx,
+                           __bf16* __restrict__ hb, int ldb, __bf16* __restrict__ ht, int ldt, int cols_p) {
+  const long long per = (long long)ldt * cols;
+  for (long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x; e < per * steps;
+       e += (long long)gridDim.x * blockDim.x) {
+    const int s = (int)(e / per), r = (int)(e % per / cols), c = (int)(e % cols);
+    const long long q = (long long)s * batch + r;
+    const __bf16 v = to_bf16(r < batch && q < n ? X[(size_t)(idx ? idx[q] : q) * cols + c] : 0.f);
+    hb[((size_t)s * ldt + r) * ldb + c] = v;
+    ht[((size_t)s * cols_p + c) * ldt + r] = v;
+  }
+}
+// x (rows x cols, FP32) -> BF16 with leading dimension ld (transposed if tr)
+__global__ void to_bf16_padded(int rows, int cols, const float* __restrict__ x, __bf16* __restrict__ y, int ld, int tr) {
   for (long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x; e < (long long)rows * cols;
        e += (long long)gridDim.x * blockDim.x) {
     const int r = (int)(e / cols), c = (int)(e % cols);
-    const float v = src[(long long)idx[r] * cols + c];
-    dst[e] = v;
-    if (dstb) dstb[e] = to_bf16(v);
-  }
-}
-
-// weighted squared error: loss partials per block, dY = 2 w (Y - T) / batch
-__global__ __launch_bounds__(256) void mse_grad(const float* __restrict__ Y, const float* __restrict__ T,
-                                                const float* __restrict__ wout, int rows, int cols,
-                                                float* __restrict__ dY, __bf16* __restrict__ dYb,
-                                                double* __restrict__ part) {
-  double acc = 0.0;
-  for (long long e = blockIdx.x * 256ll + threadIdx.x; e < (long long)rows * cols; e += (long long)gridDim.x * 256) {
-    const int c = (int)(e % cols);
-    const float d = Y[e] - T[e];
-    const float wv = wout[c];
-    acc += (double)wv * (double)d * (double)d;
-    const float g = 2.f * wv * d / (float)rows;
-    dY[e] = g;
-    dYb[e] = to_bf16(g);
-  }
-  __shared__ double red[4];
-  acc = wave_sum(acc);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
-  __syncthreads();
-  if (threadIdx.x == 0) part[blockIdx.x] = ((red[0] + red[1]) + red[2]) + red[3];
-}
-
-// dZ = dH * (Z > 0), in FP32 and BF16
-__global__ void relu_back(const float* __restrict__ dH, const float* __restrict__ Z, long long n,
-                          float* __restrict__ dZ, __bf16* __restrict__ dZb) {
-  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
-    const float g = Z[i] > 0.f ? dH[i] : 0.f;
-    dZ[i] = g;
-    dZb[i] = to_bf16(g);
-  }
-}
-
-// db[n] = sum over rows of dZ[r][n] (rows in order)
-__global__ void col_sum(const float* __restrict__ dZ, int rows, int cols, float* __restrict__ db) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= cols) return;
-  float s = 0.f;
-  for (int r = 0; r < rows; r++) s += dZ[(long long)r * cols + c];
-  db[c] = s;
-}
-
-// Adam on the FP32 master parameters
-__global__ void adam_step(float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m,
-                          float* __restrict__ v, long long n, float lr, float b1, float b2, float eps, float c1,
-                          float c2) {
-  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
-    const float gi = g[i];
-    const float mi = b1 * m[i] + (1.f - b1) * gi;
-    const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
-    m[i] = mi;
-    v[i] = vi;
-    p[i] = p[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+    y[tr ? (size_t)c * ld + r : (size_t)r * ld + c] = to_bf16(x[e]);
   }
 }
 
@@ -176,15 +339,21 @@ struct mpcx_mlp {
   std::vector<long long> woff, boff;  // offsets of W_l and b_l in the flat parameter vector
   long long nparam = 0;
   float *p = nullptr, *g = nullptr, *m = nullptr, *v = nullptr;
-  __bf16* pb = nullptr;               // BF16 copy of the parameters (GEMM operands)
-  int cap = 0;                        // batch capacity of the activation buffers
-  std::vector<float*> H, Z, dH;       // activations per layer (H[0] = input)
-  std::vector<__bf16*> Hb, dZb;
-  float* dZ = nullptr;
-  double* part = nullptr;
+  std::vector<__bf16*> w, wt;         // BF16 copies of W_l: (up32(n_next) x up32(n_prev)) and transposed
+  // forward buffers (fcap rows): activations BF16 by row, the output in FP32
+  int fcap = 0;
+  std::vector<__bf16*> Fb;
+  float *Fx = nullptr, *Fy = nullptr;
+  // training buffers (cap rows a batch)
+  int cap = 0;
+  std::vector<Act> H, dZ;             // H[0]: the input rows of a whole epoch's batches
+  long long in_rows = 0;              // rows H[0] holds
+  double *part = nullptr, *loss = nullptr;
+  long long part_n = 0, loss_n = 0;
   int* idx = nullptr;
+  long long idx_n = 0;
   float *X = nullptr, *T = nullptr, *W = nullptr;   // dataset on the device
-  long long ndata = 0;
+  long long x_n = 0, t_n = 0;
   hipStream_t st = nullptr;
   long long t = 0;                    // Adam step counter
   double gemm_ms = 0;
@@ -197,89 +366,133 @@ struct mpcx_mlp {
     if (_r != hipSuccess) return set_error(MPCX_E_HIP, hipGetErrorString(_r)); \
   } while (0)
 
-static void gemm(hipStream_t st, int M, int N, int K, const __bf16* A, long long am, long long ak, const __bf16* B,
-                 long long bk, long long bn, float* C, long long ldc, const float* bias, int relu, float* Z,
-                 __bf16* Cb, int acc) {
-  dim3 grid((N + BN - 1) / BN, (M + BM - 1) / BM);
-  hipLaunchKernelGGL(gemm_bf16, grid, dim3(GT), 0, st, M, N, K, A, am, ak, B, bk, bn, C, ldc, bias, relu, Z, Cb, acc);
-}
+static inline unsigned blocks_for(long long n) { return (unsigned)std::min<long long>((n + 255) / 256, 4096); }
 
-static int mlp_alloc_batch(mpcx_mlp* e, int batch) {
-  if (batch <= e->cap) return 0;
-  auto fr = [](void* q) { if (q) (void)hipFree(q); };
-  for (auto q : e->H) fr(q);
-  for (auto q : e->Z) fr(q);
-  for (auto q : e->dH) fr(q);
-  for (auto q : e->Hb) fr(q);
-  for (auto q : e->dZb) fr(q);
-  fr(e->dZ); fr(e->part); fr(e->idx);
-  const int L = (int)e->dims.size();
-  e->H.assign(L, nullptr); e->Z.assign(L, nullptr); e->dH.assign(L, nullptr);
-  e->Hb.assign(L, nullptr); e->dZb.assign(L, nullptr);
-  int maxd = 0;
-  for (int l = 0; l < L; l++) {
-    const size_t n = (size_t)batch * e->dims[l];
-    maxd = std::max(maxd, e->dims[l]);
-    MLCHK(hipMalloc(&e->H[l], n * 4)); MLCHK(hipMalloc(&e->Z[l], n * 4)); MLCHK(hipMalloc(&e->dH[l], n * 4));
-    MLCHK(hipMalloc(&e->Hb[l], n * 2)); MLCHK(hipMalloc(&e->dZb[l], n * 2));
-  }
-  MLCHK(hipMalloc(&e->dZ, (size_t)batch * maxd * 4));
-  MLCHK(hipMalloc(&e->part, 1024 * 8));
-  MLCHK(hipMalloc(&e->idx, (size_t)batch * 4));
-  e->cap = batch;
+template <typename T>
+static void release(T*& q) {
+  if (q) (void)hipFree(q);
+  q = nullptr;
+}
+// a buffer of at least n elements; a new one is all zeros (padding is never written)
+template <typename T>
+static int grow(hipStream_t st, T*& q, long long& have, long long n) {
+  if (n <= have) return 0;
+  release(q);
+  have = 0;
+  MLCHK(hipMalloc(&q, (size_t)n * sizeof(T)));
+  MLCHK(hipMemsetAsync(q, 0, (size_t)n * sizeof(T), st));
+  have = n;
+  return 0;
+}
+template <typename T>
+static int zeroed(hipStream_t st, T*& q, size_t n) {
+  long long have = 0;
+  return grow(st, q, have, (long long)n);
+}
+static void release_act(Act& a) { release(a.f); release(a.b); release(a.t); }
+static int make_act(hipStream_t st, Act& a, long long rows, int ldt, int cols) {
+  int rc;
+  a.cols = cols; a.ldb = up32(cols); a.ldt = ldt;
+  if ((rc = zeroed(st, a.f, (size_t)rows * cols)) || (rc = zeroed(st, a.b, (size_t)rows * a.ldb)) ||
+      (rc = zeroed(st, a.t, (size_t)a.ldb * rows)))
+    return rc;
   return 0;
 }
 
-// forward pass of `rows` rows already in H[0]/Hb[0]; output in H[L-1]
-static void mlp_forward(mpcx_mlp* e, int rows) {
-  const int L = (int)e->dims.size();
-  for (int l = 0; l + 1 < L; l++) {
-    const int K = e->dims[l], N = e->dims[l + 1];
-    const bool last = (l + 2 == L);
-    // Z = H W^T + b: W_l is (N x K) row-major, so B[k][n] = W[n*K + k]
-    gemm(e->st, rows, N, K, e->Hb[l], K, 1, e->pb + e->woff[l], 1, K, e->H[l + 1], N, e->p + e->boff[l],
-         last ? 0 : 1, e->Z[l + 1], e->Hb[l + 1], 0);
-    e->gemm_flops += 2ll * rows * N * K;
+// training buffers for batches of `batch` rows, `steps` of them an epoch
+static int train_buffers(mpcx_mlp* e, int batch, long long steps) {
+  const int L = (int)e->dims.size(), R = up32(batch);
+  int rc;
+  if (batch > e->cap) {
+    for (auto& a : e->H) release_act(a);
+    for (auto& a : e->dZ) release_act(a);
+    e->H.assign(L, Act{}); e->dZ.assign(L, Act{});
+    e->cap = 0;
+    e->in_rows = 0;
+    for (int l = 1; l < L; l++) {
+      if (l + 1 < L && (rc = make_act(e->st, e->H[l], R, R, e->dims[l]))) return rc;
+      if ((rc = make_act(e->st, e->dZ[l], R, R, e->dims[l]))) return rc;
+    }
+    e->cap = batch;
   }
+  const int ldt = up32(e->cap);
+  if (ldt * steps > e->in_rows) {
+    release_act(e->H[0]);
+    e->H[0] = Act{};
+    e->H[0].cols = e->n_in; e->H[0].ldb = up32(e->n_in); e->H[0].ldt = ldt;
+    e->in_rows = 0;
+    if ((rc = zeroed(e->st, e->H[0].b, (size_t)ldt * steps * e->H[0].ldb)) ||
+        (rc = zeroed(e->st, e->H[0].t, (size_t)ldt * steps * e->H[0].ldb)))
+      return rc;
+    e->in_rows = ldt * steps;
+  }
+  const long long tiles = (long long)(ldt / 16) * ((e->n_out + 15) / 16) + 4;
+  if ((rc = grow(e->st, e->part, e->part_n, tiles * steps))) return rc;
+  return 0;
 }
 
-// backward pass from dY (dZ of the output layer, in dZb[L-1] and dZ); gradients into g
-static void mlp_backward(mpcx_mlp* e, int rows) {
-  const int L = (int)e->dims.size();
-  for (int l = L - 2; l >= 0; l--) {
-    const int K = e->dims[l], N = e->dims[l + 1];
-    // dW_l = dZ^T H_l : (N x rows)(rows x K)
-    gemm(e->st, N, K, rows, e->dZb[l + 1], 1, N, e->Hb[l], K, 1, e->g + e->woff[l], K, nullptr, 0, nullptr, nullptr, 0);
-    hipLaunchKernelGGL(col_sum, dim3((N + 255) / 256), dim3(256), 0, e->st, (const float*)e->dH[l + 1], rows, N,
-                       e->g + e->boff[l]);
-    e->gemm_flops += 2ll * rows * N * K;
-    if (l == 0) break;
-    // dH_l = dZ W_l : (rows x N)(N x K), then dZ_l = dH_l * relu'(Z_l)
-    gemm(e->st, rows, K, N, e->dZb[l + 1], N, 1, e->pb + e->woff[l], K, 1, e->dZ, K, nullptr, 0, nullptr, nullptr, 0);
-    e->gemm_flops += 2ll * rows * N * K;
-    const long long n = (long long)rows * K;
-    hipLaunchKernelGGL(relu_back, dim3((unsigned)std::min<long long>((n + 255) / 256, 4096)), dim3(256), 0, e->st,
-                       (const float*)e->dZ, (const float*)e->Z[l], n, e->dH[l], e->dZb[l]);
+// one training step's forward and backward on batch s of the epoch's input
+// rows; the loss shares into the step's part, the gradients applied (a.on) or into g
+static void train_step(mpcx_mlp* e, int rows, long long s, const float* T, const int* idx, const float* wout, Adam a) {
+  const int L = (int)e->dims.size(), ldt = up32(e->cap), Rp = up32(rows), mt = Rp / 16;
+  hipStream_t st = e->st;
+  const __bf16* in = e->H[0].b + (size_t)s * ldt * e->H[0].ldb;
+  const __bf16* int_ = e->H[0].t + (size_t)s * ldt * e->H[0].ldb;
+  const long long tiles = (long long)(ldt / 16) * ((e->n_out + 15) / 16) + 4;
+  for (int l = 0; l + 1 < L; l++) {
+    const int K = up32(e->dims[l]), N = e->dims[l + 1], nt = (N + 15) / 16;
+    const unsigned grid = (unsigned)((mt * nt + 3) / 4);
+    const __bf16* A = l ? e->H[l].b : in;
+    if (l + 2 < L)
+      hipLaunchKernelGGL((layer_forward<1, 1>), dim3(grid), dim3(256), 0, st, rows, mt, nt, K, A, K,
+                         (const __bf16*)e->w[l], K, (const float*)(e->p + e->boff[l]), 1, e->H[l + 1]);
+    else
+      hipLaunchKernelGGL(output_loss, dim3(grid), dim3(256), 0, st, rows, mt, nt, K, A, K, (const __bf16*)e->w[l], K,
+                         (const float*)(e->p + e->boff[l]), T, idx, wout, e->dZ[l + 1], e->part + s * tiles);
+    e->gemm_flops += 2ll * rows * N * e->dims[l];
+  }
+  for (int l = L - 2; l >= 1; l--) {
+    const int K = up32(e->dims[l + 1]), N = e->dims[l], nt = (N + 15) / 16;
+    hipLaunchKernelGGL(layer_backward, dim3((unsigned)((mt * nt + 3) / 4)), dim3(256), 0, st, rows, mt, nt, K,
+                       (const __bf16*)e->dZ[l + 1].b, K, (const __bf16*)e->wt[l], K, (const float*)e->H[l].f, e->dZ[l]);
+    e->gemm_flops += 2ll * rows * N * e->dims[l + 1];
+  }
+  for (int l0 = 0; l0 + 1 < L; l0 += MAXL) {
+    GradArgs G{};
+    int blk = 0;
+    for (int l = l0; l + 1 < L && l < l0 + MAXL; l++) {
+      GradLayer& q = G.l[G.n++];
+      const int N = e->dims[l + 1], K = e->dims[l];
+      q = GradLayer{e->dZ[l + 1].t, l ? e->H[l].t : int_, e->dZ[l + 1].f, e->w[l], e->wt[l], e->woff[l], e->boff[l],
+                    N, K, up32(K), up32(N), (K + 15) / 16, blk, 0};
+      blk += ((N + 15) / 16 * q.nt + 3) / 4;
+      q.bias0 = blk;
+      blk += (N + 255) / 256;
+      e->gemm_flops += 2ll * rows * N * K;
+    }
+    hipLaunchKernelGGL(layer_grads, dim3((unsigned)blk), dim3(256), 0, st, G, rows, ldt, a, e->p, e->g, e->m, e->v);
   }
 }
 
 static void refresh_bf16(mpcx_mlp* e) {
-  hipLaunchKernelGGL(to_bf16_kernel, dim3((unsigned)std::min<long long>((e->nparam + 255) / 256, 4096)), dim3(256), 0,
-                     e->st, (const float*)e->p, e->pb, e->nparam);
+  for (size_t l = 0; l + 1 < e->dims.size(); l++)
+    hipLaunchKernelGGL(weights_bf16, dim3(blocks_for((long long)e->dims[l] * e->dims[l + 1])), dim3(256), 0, e->st,
+                       e->dims[l + 1], e->dims[l], (const float*)(e->p + e->woff[l]), e->w[l], up32(e->dims[l]), e->wt[l],
+                       up32(e->dims[l + 1]));
 }
 
 extern "C" int mpcx_mlp_destroy(mpcx_mlp* e) {
   if (!e) return 0;
   mpcx::handle_del(mpcx::H_MLP, e);
   if (e->st) (void)hipStreamSynchronize(e->st);
-  auto fr = [](void* q) { if (q) (void)hipFree(q); };
-  fr(e->p); fr(e->g); fr(e->m); fr(e->v); fr(e->pb);
-  for (auto q : e->H) fr(q);
-  for (auto q : e->Z) fr(q);
-  for (auto q : e->dH) fr(q);
-  for (auto q : e->Hb) fr(q);
-  for (auto q : e->dZb) fr(q);
-  fr(e->dZ); fr(e->part); fr(e->idx); fr(e->X); fr(e->T); fr(e->W);
+  release(e->p); release(e->g); release(e->m); release(e->v);
+  for (auto& q : e->w) release(q);
+  for (auto& q : e->wt) release(q);
+  for (auto& q : e->Fb) release(q);
+  for (auto& a : e->H) release_act(a);
+  for (auto& a : e->dZ) release_act(a);
+  release(e->Fx); release(e->Fy); release(e->part); release(e->loss); release(e->idx);
+  release(e->X); release(e->T); release(e->W);
   if (e->st) (void)hipStreamDestroy(e->st);
   delete e;
   return 0;
@@ -312,10 +525,19 @@ extern "C" int mpcx_mlp_create(mpcx_mlp** out, int32_t n_in, int32_t n_hidden, i
   }
   if (hipStreamCreateWithFlags(&e->st, hipStreamNonBlocking) != hipSuccess ||
       hipMalloc(&e->p, o * 4) != hipSuccess || hipMalloc(&e->g, o * 4) != hipSuccess ||
-      hipMalloc(&e->m, o * 4) != hipSuccess || hipMalloc(&e->v, o * 4) != hipSuccess ||
-      hipMalloc(&e->pb, o * 2) != hipSuccess) {
+      hipMalloc(&e->m, o * 4) != hipSuccess || hipMalloc(&e->v, o * 4) != hipSuccess) {
     mpcx_mlp_destroy(e);
     return set_error(MPCX_E_HIP, "device allocation failed");
+  }
+  const size_t nl = e->dims.size() - 1;
+  e->w.assign(nl, nullptr);
+  e->wt.assign(nl, nullptr);
+  for (size_t l = 0; l < nl; l++) {
+    const size_t n = (size_t)up32(e->dims[l]) * up32(e->dims[l + 1]);
+    if (zeroed(e->st, e->w[l], n) || zeroed(e->st, e->wt[l], n)) {
+      mpcx_mlp_destroy(e);
+      return MPCX_E_HIP;
+    }
   }
   MLCHK(hipMemcpy(e->p, p.data(), o * 4, hipMemcpyHostToDevice));
   MLCHK(hipMemset(e->m, 0, o * 4));
@@ -346,130 +568,162 @@ extern "C" int mpcx_mlp_set_params(mpcx_mlp* e, const float* flat) {
   return 0;
 }
 
-// rows -> H[0] (FP32 and BF16) from a host array
-static int load_rows(mpcx_mlp* e, int rows, const float* x) {
-  const size_t n = (size_t)rows * e->n_in;
-  MLCHK(hipMemcpyAsync(e->H[0], x, n * 4, hipMemcpyHostToDevice, e->st));
-  hipLaunchKernelGGL(to_bf16_kernel, dim3((unsigned)std::min<size_t>((n + 255) / 256, 4096)), dim3(256), 0, e->st,
-                     (const float*)e->H[0], e->Hb[0], (long long)n);
-  return 0;
-}
-
+// Forward pass.  32 x 32 tiles once a layer has enough of them to fill the
+// chip's 1024 SIMDs several times over (they read half as much per product),
+// 16 x 16 below that, where the number of waves is what counts.
 extern "C" int mpcx_mlp_forward(mpcx_mlp* e, int32_t rows, const float* x, float* y) {
   if (!e || rows < 1 || !x || !y) return set_error(MPCX_E_ARG, "bad arguments");
-  int rc = mlp_alloc_batch(e, rows);
-  if (rc) return rc;
-  if ((rc = load_rows(e, rows, x))) return rc;
-  mlp_forward(e, rows);
-  const int L = (int)e->dims.size();
-  MLCHK(hipMemcpyAsync(y, e->H[L - 1], (size_t)rows * e->n_out * 4, hipMemcpyDeviceToHost, e->st));
+  const int L = (int)e->dims.size(), Rp = up32(rows);
+  int rc;
+  if (rows > e->fcap) {
+    for (auto& q : e->Fb) release(q);
+    release(e->Fx); release(e->Fy);
+    e->fcap = 0;
+    e->Fb.assign(L - 1, nullptr);
+    for (int l = 0; l + 1 < L; l++)
+      if ((rc = zeroed(e->st, e->Fb[l], (size_t)Rp * up32(e->dims[l])))) return rc;
+    MLCHK(hipMalloc(&e->Fx, (size_t)rows * e->n_in * 4));
+    MLCHK(hipMalloc(&e->Fy, (size_t)rows * e->n_out * 4));
+    e->fcap = rows;
+  }
+  MLCHK(hipMemcpyAsync(e->Fx, x, (size_t)rows * e->n_in * 4, hipMemcpyHostToDevice, e->st));
+  hipLaunchKernelGGL(to_bf16_padded, dim3(blocks_for((long long)rows * e->n_in)), dim3(256), 0, e->st, rows, e->n_in,
+                     (const float*)e->Fx, e->Fb[0], up32(e->n_in), 0);
+  for (int l = 0; l + 1 < L; l++) {
+    const int K = up32(e->dims[l]), N = e->dims[l + 1];
+    const bool last = l + 2 == L;
+    const Act H{last ? e->Fy : nullptr, last ? nullptr : e->Fb[l + 1], nullptr, N, up32(N), 0};
+    const bool big = (long long)(Rp / 16) * ((N + 15) / 16) >= 4096;
+    const int mt = Rp / (big ? 32 : 16), nt = big ? up32(N) / 32 : (N + 15) / 16;
+    const dim3 grid((unsigned)(((long long)mt * nt + 3) / 4));
+    auto launch = [&](auto k) {
+      hipLaunchKernelGGL(k, grid, dim3(256), 0, e->st, (int)rows, mt, nt, K, (const __bf16*)e->Fb[l], K,
+                         (const __bf16*)e->w[l], K, (const float*)(e->p + e->boff[l]), last ? 0 : 1, H);
+    };
+    if (big) launch(layer_forward<2, 2>);
+    else launch(layer_forward<1, 1>);
+    e->gemm_flops += 2ll * rows * N * e->dims[l];
+  }
+  MLCHK(hipMemcpyAsync(y, e->Fy, (size_t)rows * e->n_out * 4, hipMemcpyDeviceToHost, e->st));
   MLCHK(hipStreamSynchronize(e->st));
   return 0;
 }
 
-// loss and gradient of one batch held in H[0] with targets T (device)
-static int loss_grad(mpcx_mlp* e, int rows, const float* Td, const float* wd, double* loss) {
-  const int L = (int)e->dims.size();
-  mlp_forward(e, rows);
-  const long long n = (long long)rows * e->n_out;
-  const int nb = (int)std::min<long long>((n + 255) / 256, 1024);
-  hipLaunchKernelGGL(mse_grad, dim3(nb), dim3(256), 0, e->st, (const float*)e->H[L - 1], Td, wd, rows, e->n_out,
-                     e->dH[L - 1], e->dZb[L - 1], e->part);
-  mlp_backward(e, rows);
-  std::vector<double> part(nb);
-  MLCHK(hipMemcpyAsync(part.data(), e->part, nb * 8, hipMemcpyDeviceToHost, e->st));
-  MLCHK(hipStreamSynchronize(e->st));
-  double s = 0.0;
-  for (int b = 0; b < nb; b++) s += part[b];
-  *loss = s / rows;
+// dataset rows, targets and output weights on the device
+static int upload_data(mpcx_mlp* e, long long n, const float* x, const float* target, const float* wout) {
+  int rc;
+  long long w_n = e->W ? e->n_out : 0;
+  if ((rc = grow(e->st, e->X, e->x_n, n * e->n_in)) || (rc = grow(e->st, e->T, e->t_n, n * e->n_out)) ||
+      (rc = grow(e->st, e->W, w_n, e->n_out)))
+    return rc;
+  MLCHK(hipMemcpyAsync(e->X, x, (size_t)n * e->n_in * 4, hipMemcpyHostToDevice, e->st));
+  MLCHK(hipMemcpyAsync(e->T, target, (size_t)n * e->n_out * 4, hipMemcpyHostToDevice, e->st));
+  MLCHK(hipMemcpyAsync(e->W, wout, (size_t)e->n_out * 4, hipMemcpyHostToDevice, e->st));
   return 0;
 }
+static void launch_inputs(mpcx_mlp* e, long long n, int batch, long long steps, const int* idx) {
+  const Act& a = e->H[0];
+  hipLaunchKernelGGL(input_rows, dim3(blocks_for((long long)a.ldt * a.cols * steps)), dim3(256), 0, e->st, (int)n, batch,
+                     (int)steps, a.cols, (const float*)e->X, idx, a.b, a.ldb, a.t, a.ldt, a.ldb);
+}
+static void launch_loss(mpcx_mlp* e, int tiles, long long steps, double* out) {
+  const long long stride = (long long)(up32(e->cap) / 16) * ((e->n_out + 15) / 16) + 4;
+  hipLaunchKernelGGL(loss_sums, dim3((unsigned)steps), dim3(64), 0, e->st, tiles, stride, (const double*)e->part, out);
+}
+static int loss_tiles(const mpcx_mlp* e, int rows) { return (up32(rows) / 16) * ((e->n_out + 15) / 16); }
 
 extern "C" int mpcx_mlp_loss_grad(mpcx_mlp* e, int32_t rows, const float* x, const float* target, const float* wout,
                                   double* loss, float* grad) {
   if (!e || rows < 1 || !x || !target || !wout || !loss) return set_error(MPCX_E_ARG, "bad arguments");
-  int rc = mlp_alloc_batch(e, rows);
-  if (rc) return rc;
-  float *Td = nullptr, *wd = nullptr;
-  MLCHK(hipMalloc(&Td, (size_t)rows * e->n_out * 4));
-  MLCHK(hipMalloc(&wd, (size_t)e->n_out * 4));
-  MLCHK(hipMemcpyAsync(Td, target, (size_t)rows * e->n_out * 4, hipMemcpyHostToDevice, e->st));
-  MLCHK(hipMemcpyAsync(wd, wout, (size_t)e->n_out * 4, hipMemcpyHostToDevice, e->st));
-  if ((rc = load_rows(e, rows, x)) == 0) rc = loss_grad(e, rows, Td, wd, loss);
-  if (rc == 0 && grad) {
-    if (hipMemcpy(grad, e->g, e->nparam * 4, hipMemcpyDeviceToHost) != hipSuccess)
-      rc = set_error(MPCX_E_HIP, "hipMemcpy failed");
-  }
-  (void)hipFree(Td);
-  (void)hipFree(wd);
-  return rc;
+  int rc;
+  if ((rc = train_buffers(e, rows, 1)) || (rc = upload_data(e, rows, x, target, wout)) ||
+      (rc = grow(e->st, e->loss, e->loss_n, 1)))
+    return rc;
+  launch_inputs(e, rows, rows, 1, nullptr);
+  train_step(e, rows, 0, e->T, nullptr, e->W, Adam{});
+  launch_loss(e, loss_tiles(e, rows), 1, e->loss);
+  MLCHK(hipMemcpyAsync(loss, e->loss, 8, hipMemcpyDeviceToHost, e->st));
+  if (grad) MLCHK(hipMemcpyAsync(grad, e->g, e->nparam * 4, hipMemcpyDeviceToHost, e->st));
+  MLCHK(hipStreamSynchronize(e->st));
+  *loss = *loss / rows;
+  return 0;
 }
 
 // Minibatch Adam over a dataset held on the device.  Each epoch visits the n
 // rows in an order shuffled by a 64-bit LCG seeded with `seed` and the epoch.
+// The host only makes the orders, a few epochs at a time, and launches: the
+// losses stay on the device until the end of the run (waiting for each
+// minibatch's, the allocations and 21 launches a step, took 460 us a step).
 extern "C" int mpcx_mlp_train(mpcx_mlp* e, int64_t n, const float* x, const float* target, const float* wout,
                               int32_t batch, int32_t epochs, float lr, uint64_t seed, double* epoch_loss) {
   if (!e || n < 1 || !x || !target || !wout || batch < 1 || epochs < 0) return set_error(MPCX_E_ARG, "bad arguments");
-  int rc = mlp_alloc_batch(e, batch);
-  if (rc) return rc;
-  auto fr = [](void* q) { if (q) (void)hipFree(q); };
-  fr(e->X); fr(e->T); fr(e->W);
-  e->X = e->T = e->W = nullptr;
-  MLCHK(hipMalloc(&e->X, (size_t)n * e->n_in * 4));
-  MLCHK(hipMalloc(&e->T, (size_t)n * e->n_out * 4));
-  MLCHK(hipMalloc(&e->W, (size_t)e->n_out * 4));
-  MLCHK(hipMemcpy(e->X, x, (size_t)n * e->n_in * 4, hipMemcpyHostToDevice));
-  MLCHK(hipMemcpy(e->T, target, (size_t)n * e->n_out * 4, hipMemcpyHostToDevice));
-  MLCHK(hipMemcpy(e->W, wout, (size_t)e->n_out * 4, hipMemcpyHostToDevice));
-  e->ndata = n;
-  float* Tb = nullptr;
-  MLCHK(hipMalloc(&Tb, (size_t)batch * e->n_out * 4));
-  std::vector<int> order(n);
+  batch = (int32_t)std::min<int64_t>(batch, n);
+  const long long steps = (n + batch - 1) / batch;
+  const int CHUNK = (int)std::max<int64_t>(1, std::min<int64_t>(64, (1 << 22) / n));   // epochs whose orders are uploaded together
+  int rc;
+  if ((rc = train_buffers(e, batch, steps)) || (rc = upload_data(e, n, x, target, wout)) ||
+      (rc = grow(e->st, e->idx, e->idx_n, n * CHUNK)) || (rc = grow(e->st, e->loss, e->loss_n, steps * std::max(epochs, 1))))
+    return rc;
+  std::vector<int> order((size_t)n * std::min(CHUNK, std::max(epochs, 1)));
   hipEvent_t a0, a1;
   (void)hipEventCreate(&a0);
   (void)hipEventCreate(&a1);
   (void)hipEventRecord(a0, e->st);
   e->gemm_flops = 0;
-  for (int ep = 0; ep < epochs; ep++) {
-    for (long long i = 0; i < n; i++) order[i] = (int)i;
-    unsigned long long s = (seed + 1) * 6364136223846793005ull + (unsigned long long)ep * 1442695040888963407ull;
-    for (long long i = n - 1; i > 0; i--) {   // Fisher-Yates
-      s = s * 6364136223846793005ull + 1442695040888963407ull;
-      const long long j = (long long)((s >> 33) % (unsigned long long)(i + 1));
-      std::swap(order[i], order[j]);
+  const int tail = (int)(n - (steps - 1) * batch);
+  for (int e0 = 0; e0 < epochs && !rc; e0 += CHUNK) {
+    const int ne = std::min(CHUNK, epochs - e0);
+    if (e0) rc = hipStreamSynchronize(e->st) == hipSuccess ? 0 : set_error(MPCX_E_HIP, "hipStreamSynchronize failed");
+    for (int q = 0; q < ne; q++) {
+      int* o = order.data() + (size_t)q * n;
+      for (long long i = 0; i < n; i++) o[i] = (int)i;
+      unsigned long long s = (seed + 1) * 6364136223846793005ull + (unsigned long long)(e0 + q) * 1442695040888963407ull;
+      for (long long i = n - 1; i > 0; i--) {   // Fisher-Yates
+        s = s * 6364136223846793005ull + 1442695040888963407ull;
+        const long long j = (long long)((s >> 33) % (unsigned long long)(i + 1));
+        std::swap(o[i], o[j]);
+      }
     }
-    double tot = 0.0;
-    long long seen = 0;
-    for (long long b0 = 0; b0 < n; b0 += batch) {
-      const int rows = (int)std::min<long long>(batch, n - b0);
-      MLCHK(hipMemcpyAsync(e->idx, order.data() + b0, rows * 4, hipMemcpyHostToDevice, e->st));
-      hipLaunchKernelGGL(gather_rows, dim3(64), dim3(256), 0, e->st, (const float*)e->X, (const int*)e->idx, rows,
-                         e->n_in, e->H[0], e->Hb[0]);
-      hipLaunchKernelGGL(gather_rows, dim3(256), dim3(256), 0, e->st, (const float*)e->T, (const int*)e->idx, rows,
-                         e->n_out, Tb, (__bf16*)nullptr);
-      double l = 0.0;
-      if ((rc = loss_grad(e, rows, Tb, e->W, &l))) break;
-      tot += l * rows;
-      seen += rows;
-      e->t += 1;
-      const float c1 = 1.f - powf(0.9f, (float)e->t), c2 = 1.f - powf(0.999f, (float)e->t);
-      hipLaunchKernelGGL(adam_step, dim3((unsigned)std::min<long long>((e->nparam + 255) / 256, 4096)), dim3(256), 0,
-                         e->st, e->p, (const float*)e->g, e->m, e->v, e->nparam, lr, 0.9f, 0.999f, 1e-8f, c1, c2);
-      refresh_bf16(e);
+    if (!rc && hipMemcpyAsync(e->idx, order.data(), (size_t)ne * n * 4, hipMemcpyHostToDevice, e->st) != hipSuccess)
+      rc = set_error(MPCX_E_HIP, "hipMemcpyAsync failed");
+    for (int q = 0; q < ne && !rc; q++) {
+      const int* idx = e->idx + (size_t)q * n;
+      double* lo = e->loss + (size_t)(e0 + q) * steps;
+      launch_inputs(e, n, batch, steps, idx);
+      for (long long s = 0; s < steps; s++) {
+        e->t += 1;
+        const float c1 = 1.f - powf(0.9f, (float)e->t), c2 = 1.f - powf(0.999f, (float)e->t);
+        train_step(e, s + 1 < steps ? batch : tail, s, e->T, idx + s * batch, e->W,
+                   Adam{lr, 0.9f, 0.999f, 1e-8f, c1, c2, 1});
+      }
+      if (steps > 1) launch_loss(e, loss_tiles(e, batch), steps - 1, lo);
+      hipLaunchKernelGGL(loss_sums, dim3(1), dim3(64), 0, e->st, loss_tiles(e, tail), 0ll,
+                         (const double*)(e->part + (steps - 1) * ((long long)(up32(e->cap) / 16) * ((e->n_out + 15) / 16) + 4)),
+                         lo + steps - 1);
     }
-    if (rc) break;
-    if (epoch_loss) epoch_loss[ep] = tot / (double)seen;
   }
   (void)hipEventRecord(a1, e->st);
-  (void)hipEventSynchronize(a1);
+  std::vector<double> loss((size_t)steps * std::max(epochs, 1));
+  if (!rc && epochs > 0 &&
+      hipMemcpyAsync(loss.data(), e->loss, (size_t)steps * epochs * 8, hipMemcpyDeviceToHost, e->st) != hipSuccess)
+    rc = set_error(MPCX_E_HIP, "hipMemcpyAsync failed");
+  const hipError_t sr = hipStreamSynchronize(e->st);   // the orders and the caller's arrays are read until here
   float ms = 0;
   (void)hipEventElapsedTime(&ms, a0, a1);
   e->gemm_ms = ms;
   (void)hipEventDestroy(a0);
   (void)hipEventDestroy(a1);
-  (void)hipFree(Tb);
   if (rc) return rc;
-  MLCHK(hipStreamSynchronize(e->st));
+  MLCHK(sr);
+  if (epoch_loss)
+    for (int ep = 0; ep < epochs; ep++) {
+      double tot = 0.0;
+      for (long long s = 0; s < steps; s++) {
+        const int rows = s + 1 < steps ? batch : tail;
+        tot += loss[(size_t)ep * steps + s] / rows * rows;
+      }
+      epoch_loss[ep] = tot / (double)n;
+    }
   return 0;
 }
 
@@ -486,21 +740,32 @@ extern "C" int mpcx_mlp_train_stats(mpcx_mlp* e, double* ms, double* gemm_flops)
 extern "C" int mpcx_gemm_bf16(int32_t M, int32_t N, int32_t K, const float* A, const float* B, float* C, int32_t reps,
                               double* ms) {
   if (M < 1 || N < 1 || K < 1 || !A || !B || !C || reps < 1) return set_error(MPCX_E_ARG, "bad arguments");
+  const int Mp = up32(M), Np = up32(N), Kp = up32(K);
   float *Af = nullptr, *Bf = nullptr, *Cd = nullptr;
   __bf16 *Ab = nullptr, *Bb = nullptr;
   MLCHK(hipMalloc(&Af, (size_t)M * K * 4)); MLCHK(hipMalloc(&Bf, (size_t)K * N * 4));
-  MLCHK(hipMalloc(&Ab, (size_t)M * K * 2)); MLCHK(hipMalloc(&Bb, (size_t)K * N * 2));
+  MLCHK(hipMalloc(&Ab, (size_t)Mp * Kp * 2)); MLCHK(hipMalloc(&Bb, (size_t)Np * Kp * 2));
   MLCHK(hipMalloc(&Cd, (size_t)M * N * 4));
+  MLCHK(hipMemset(Ab, 0, (size_t)Mp * Kp * 2));
+  MLCHK(hipMemset(Bb, 0, (size_t)Np * Kp * 2));
   MLCHK(hipMemcpy(Af, A, (size_t)M * K * 4, hipMemcpyHostToDevice));
   MLCHK(hipMemcpy(Bf, B, (size_t)K * N * 4, hipMemcpyHostToDevice));
-  hipLaunchKernelGGL(to_bf16_kernel, dim3(1024), dim3(256), 0, 0, (const float*)Af, Ab, (long long)M * K);
-  hipLaunchKernelGGL(to_bf16_kernel, dim3(1024), dim3(256), 0, 0, (const float*)Bf, Bb, (long long)K * N);
+  hipLaunchKernelGGL(to_bf16_padded, dim3(1024), dim3(256), 0, 0, M, K, (const float*)Af, Ab, Kp, 0);
+  hipLaunchKernelGGL(to_bf16_padded, dim3(1024), dim3(256), 0, 0, K, N, (const float*)Bf, Bb, Kp, 1);
   hipEvent_t a0, a1;
   (void)hipEventCreate(&a0);
   (void)hipEventCreate(&a1);
-  gemm(0, M, N, K, Ab, K, 1, Bb, N, 1, Cd, N, nullptr, 0, nullptr, nullptr, 0);
+  const bool big = (long long)(Mp / 16) * ((N + 15) / 16) >= 4096;
+  const int mt = Mp / (big ? 32 : 16), nt = big ? Np / 32 : (N + 15) / 16;
+  const Act C_{Cd, nullptr, nullptr, N, 0, 0};
+  auto product = [&](auto k) {
+    hipLaunchKernelGGL(k, dim3((unsigned)(((long long)mt * nt + 3) / 4)), dim3(256), 0, 0, (int)M, mt, nt, Kp,
+                       (const __bf16*)Ab, Kp, (const __bf16*)Bb, Kp, (const float*)nullptr, 0, C_);
+  };
+  auto once = [&] { if (big) product(layer_forward<2, 2>); else product(layer_forward<1, 1>); };
+  once();
   (void)hipEventRecord(a0, 0);
-  for (int r = 0; r < reps; r++) gemm(0, M, N, K, Ab, K, 1, Bb, N, 1, Cd, N, nullptr, 0, nullptr, nullptr, 0);
+  for (int r = 0; r < reps; r++) once();
   (void)hipEventRecord(a1, 0);
   hipError_t rr = hipEventSynchronize(a1);
   float t = 0;
