@@ -27,6 +27,7 @@
 #include <algorithm>
 #include "mpcx_device.h"
 #include "mpcx_host.h"
+#include "mpcx_stage.h"
 #include "mpcx_kernels.h"
 #include "../../include/mpcx.h"
 
@@ -3467,13 +3468,10 @@ extern "C" int mpcx_co_set_state(mpcx_co* e, int32_t cstep, const double* x, con
   const size_t NT = (size_t)e->P.NT, nd = (size_t)e->nd;
   CoD& D = e->D;
   if (solvent) {
-    HIPCHK(hipMemcpy(D.x, x, NT * 8, hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(D.y, y, NT * 8, hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(D.z, z, NT * 8, hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(D.vx, vx, NT * 8, hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(D.vy, vy, NT * 8, hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(D.vz, vz, NT * 8, hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(D.flag, flag, NT * 4, hipMemcpyHostToDevice));
+    const int rc = mpcx::copy_in({mpcx::upload(D.x, x, NT * 8), mpcx::upload(D.y, y, NT * 8), mpcx::upload(D.z, z, NT * 8),
+                                  mpcx::upload(D.vx, vx, NT * 8), mpcx::upload(D.vy, vy, NT * 8),
+                                  mpcx::upload(D.vz, vz, NT * 8), mpcx::upload(D.flag, flag, NT * 4)}, e->st);
+    if (rc) return rc;
   }
   std::vector<double> dim(12 * MAXSG, 0.0);
   const double* src[9] = {xd, yd, zd, vxd, vyd, vzd, fxd, fyd, fzd};
@@ -4102,13 +4100,9 @@ extern "C" int mpcx_co_get_state(mpcx_co* e, double* x, double* y, double* z, do
   HIPCHK(hipStreamSynchronize(e->st));
   const size_t NT = (size_t)e->P.NT;
   CoD& D = e->D;
-  if (x) HIPCHK(hipMemcpy(x, D.x, NT * 8, hipMemcpyDeviceToHost));
-  if (y) HIPCHK(hipMemcpy(y, D.y, NT * 8, hipMemcpyDeviceToHost));
-  if (z) HIPCHK(hipMemcpy(z, D.z, NT * 8, hipMemcpyDeviceToHost));
-  if (vx) HIPCHK(hipMemcpy(vx, D.vx, NT * 8, hipMemcpyDeviceToHost));
-  if (vy) HIPCHK(hipMemcpy(vy, D.vy, NT * 8, hipMemcpyDeviceToHost));
-  if (vz) HIPCHK(hipMemcpy(vz, D.vz, NT * 8, hipMemcpyDeviceToHost));
-  if (flag) HIPCHK(hipMemcpy(flag, D.flag, NT * 4, hipMemcpyDeviceToHost));
+  const int rc = mpcx::copy_out({{x, D.x, NT * 8}, {y, D.y, NT * 8}, {z, D.z, NT * 8}, {vx, D.vx, NT * 8}, {vy, D.vy, NT * 8},
+                                 {vz, D.vz, NT * 8}, {flag, D.flag, NT * 4}}, e->st);
+  if (rc) return rc;
   if (dimer12) {
     std::vector<double> dim(12 * MAXSG);
     HIPCHK(hipMemcpy(dim.data(), D.dim, dim.size() * 8, hipMemcpyDeviceToHost));

@@ -7,6 +7,7 @@
 #include <stdint.h>
 #include "mpcx_device.h"
 #include "mpcx_host.h"
+#include "mpcx_stage.h"
 #include "../../include/mpcx.h"
 
 namespace mpcx {
@@ -42,7 +43,11 @@ extern "C" int mpcx_shutdown(void) {
   for (void* p : live[mpcx::H_SK]) (void)mpcx_sk_destroy((mpcx_sk*)p);
   for (void* p : live[mpcx::H_MLP]) (void)mpcx_mlp_destroy((mpcx_mlp*)p);
   int n = 0;
-  if (hipGetDeviceCount(&n) == hipSuccess && n > 0) (void)hipDeviceSynchronize();
+  if (hipGetDeviceCount(&n) == hipSuccess && n > 0) {
+    (void)hipDeviceSynchronize();
+    mpcx::blocks_release();
+    mpcx::stage_release();
+  }
   return 0;
 }
 

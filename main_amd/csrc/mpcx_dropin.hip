@@ -11,6 +11,8 @@
 #include <vector>
 #include "mpcx_device.h"
 #include "mpcx_host.h"
+#include "mpcx_stage.h"
+#include "mpcx_kernels.h"
 #include "../../include/mpcx.h"
 
 #pragma clang fp contract(off)
@@ -22,13 +24,15 @@ constexpr int BT = 256;
 constexpr int CB = 1024;   // elements per block of the compaction scans
 
 // -------------------------------------------------------------- device buffers
+// (kept between calls: 18 hipMalloc and hipFree a call, each a wait for the
+// device, were a quarter of a collision's time at 270,000 particles)
 struct Buf {
   void* p = nullptr;
   size_t n = 0;
-  ~Buf() { if (p) (void)hipFree(p); }
+  ~Buf() { block_put(p, n); }
   bool alloc(size_t bytes) {
-    n = bytes;
-    return hipMalloc(&p, bytes ? bytes : 8) == hipSuccess;
+    p = block_get(bytes, &n);
+    return p != nullptr;
   }
   template <typename T> T* as() { return (T*)p; }
 };
@@ -43,6 +47,20 @@ static int up(Buf& b, const void* h, size_t bytes) {
   if (!b.alloc(bytes)) return set_error(MPCX_E_HIP, "hipMalloc failed");
   if (h && bytes) DCHK(hipMemcpy(b.p, h, bytes, hipMemcpyHostToDevice));
   return 0;
+}
+// buffers for several arrays, uploaded together
+struct Up {
+  Buf* b;
+  const void* h;
+  size_t bytes;
+};
+static int up_all(const std::vector<Up>& v) {
+  std::vector<HostCopy> cp;
+  for (const Up& u : v) {
+    if (!u.b->alloc(u.bytes)) return set_error(MPCX_E_HIP, "hipMalloc failed");
+    if (u.h) cp.push_back(upload(u.b->p, u.h, u.bytes));
+  }
+  return copy_in(cp, 0);
 }
 static int down(void* h, Buf& b, size_t bytes) {
   if (h && bytes) DCHK(hipMemcpy(h, b.p, bytes, hipMemcpyDeviceToHost));
@@ -109,12 +127,15 @@ __global__ void k_cell_cm(long long numcell, const int* cnt, const int* off, int
   uvx[c] = st * cp; uvy[c] = st * sp; uvz[c] = th;
 }
 // mpc_rotation_mod.f95:205-230
-__global__ void k_rotate(int NT, const long long* ncn, const double* vxcm, const double* vycm, const double* vzcm,
+// (a particle whose cell is out of range raised an error in k_cells: the call
+// then returns without an output)
+__global__ void k_rotate(int NT, long long numcell, const long long* ncn, const double* vxcm, const double* vycm, const double* vzcm,
                          const double* uvx, const double* uvy, const double* uvz, double cr, double sr,
                          double* vx, double* vy, double* vz) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= NT) return;
   long long c = ncn[i] - 1;
+  if (c < 0 || c >= numcell) return;
   double ux = uvx[c], uy = uvy[c], uz = uvz[c], cx = vxcm[c], cy = vycm[c], cz = vzcm[c];
   double omc = 1.0 - cr;
   double dx = vx[i] - cx, dy = vy[i] - cy, dz = vz[i] - cz;
@@ -316,13 +337,12 @@ extern "C" int mpcx_mpc_rotation(int32_t NT, double rotang, int64_t numcell, dou
                                  const double* draws) {
   if (NT < 0 || numcell < 1 || !box || !Xsol || !draws) return set_error(MPCX_E_ARG, "bad arguments");
   const size_t n = (size_t)NT, mc = (size_t)numcell;
-  Buf x, y, z, vx, vy, vz, dr, ncn, cnt, rank, bucket, offb, cm[7], err;
+  Buf x, y, z, vx, vy, vz, dr, ncn, cnt, rank, bucket, offb, part, cm[7], err;
   int r;
-  if ((r = up(x, Xsol, n * 8)) || (r = up(y, Ysol, n * 8)) || (r = up(z, Zsol, n * 8)) ||
-      (r = up(vx, VXsol, n * 8)) || (r = up(vy, VYsol, n * 8)) || (r = up(vz, VZsol, n * 8)) ||
-      (r = up(dr, draws, (3 + 2 * mc) * 8)) || (r = up(ncn, nullptr, n * 8)) || (r = up(cnt, nullptr, mc * 4)) ||
-      (r = up(rank, nullptr, n * 4)) || (r = up(bucket, nullptr, n * 4)) || (r = up(offb, nullptr, (mc + 1) * 4)) ||
-      (r = up(err, nullptr, 4)))
+  if ((r = up_all({{&x, Xsol, n * 8}, {&y, Ysol, n * 8}, {&z, Zsol, n * 8}, {&vx, VXsol, n * 8}, {&vy, VYsol, n * 8},
+                   {&vz, VZsol, n * 8}, {&dr, draws, (3 + 2 * mc) * 8}, {&ncn, nullptr, n * 8}, {&cnt, nullptr, mc * 4},
+                   {&rank, nullptr, n * 4}, {&bucket, nullptr, n * 4}, {&offb, nullptr, (mc + 1) * 4},
+                   {&part, nullptr, (mc / 4096 + 2) * 4}, {&err, nullptr, 4}})))
     return r;
   for (auto& b : cm)
     if ((r = up(b, nullptr, mc * 8))) return r;
@@ -332,11 +352,7 @@ extern "C" int mpcx_mpc_rotation(int32_t NT, double rotang, int64_t numcell, dou
   hipLaunchKernelGGL(k_cells, dim3(nblk(n)), dim3(BT), 0, 0, NT, box[0], box[1], xs, ys, zs, x.as<double>(),
                      y.as<double>(), z.as<double>(), (long long)numcell, ncn.as<long long>(), cnt.as<int>(),
                      rank.as<int>(), err.as<int>());
-  if ((r = read_err(err))) return r;
-  std::vector<int> c(mc), off;
-  DCHK(hipMemcpy(c.data(), cnt.p, mc * 4, hipMemcpyDeviceToHost));
-  host_scan(c, off);
-  DCHK(hipMemcpy(offb.p, off.data(), (mc + 1) * 4, hipMemcpyHostToDevice));
+  launch_scan(0, cnt.as<int>(), (long long)mc, part.as<int>(), offb.as<int>());
   hipLaunchKernelGGL(k_scatter, dim3(nblk(n)), dim3(BT), 0, 0, NT, ncn.as<long long>(), rank.as<int>(),
                      offb.as<int>(), bucket.as<int>());
   const double twopi = 2.0 * (4.0 * atan(1.0));
@@ -344,16 +360,14 @@ extern "C" int mpcx_mpc_rotation(int32_t NT, double rotang, int64_t numcell, dou
                      bucket.as<int>(), vx.as<double>(), vy.as<double>(), vz.as<double>(), dr.as<double>(), twopi,
                      cm[0].as<double>(), cm[1].as<double>(), cm[2].as<double>(), cm[3].as<double>(),
                      cm[4].as<double>(), cm[5].as<double>(), cm[6].as<double>());
-  hipLaunchKernelGGL(k_rotate, dim3(nblk(n)), dim3(BT), 0, 0, NT, ncn.as<long long>(), cm[0].as<double>(),
+  hipLaunchKernelGGL(k_rotate, dim3(nblk(n)), dim3(BT), 0, 0, NT, (long long)numcell, ncn.as<long long>(), cm[0].as<double>(),
                      cm[1].as<double>(), cm[2].as<double>(), cm[4].as<double>(), cm[5].as<double>(),
                      cm[6].as<double>(), cos(rotang), sin(rotang), vx.as<double>(), vy.as<double>(),
                      vz.as<double>());
-  if ((r = down(VXsol, vx, n * 8)) || (r = down(VYsol, vy, n * 8)) || (r = down(VZsol, vz, n * 8)) ||
-      (r = down(VXCM, cm[0], mc * 8)) || (r = down(VYCM, cm[1], mc * 8)) || (r = down(VZCM, cm[2], mc * 8)) ||
-      (r = down(tCellShift, cm[3], mc * 8)) || (r = down(UVX, cm[4], mc * 8)) || (r = down(UVY, cm[5], mc * 8)) ||
-      (r = down(UVZ, cm[6], mc * 8)) || (r = down(NewCellN, ncn, n * 8)))
-    return r;
-  return 0;
+  if ((r = read_err(err))) return r;
+  return copy_out({{VXsol, vx.p, n * 8}, {VYsol, vy.p, n * 8}, {VZsol, vz.p, n * 8}, {VXCM, cm[0].p, mc * 8},
+                   {VYCM, cm[1].p, mc * 8}, {VZCM, cm[2].p, mc * 8}, {tCellShift, cm[3].p, mc * 8}, {UVX, cm[4].p, mc * 8},
+                   {UVY, cm[5].p, mc * 8}, {UVZ, cm[6].p, mc * 8}, {NewCellN, ncn.p, n * 8}}, 0);
 }
 
 extern "C" int mpcx_reaction_simple(double MPCt, int64_t numcell, double k1, int32_t NT, int32_t* flag,
@@ -376,14 +390,14 @@ extern "C" int mpcx_reaction_simple(double MPCt, int64_t numcell, double k1, int
   Buf f, tb, sb, dr, tp, err;
   int r;
   const size_t nc = (size_t)numcell;
-  if ((r = up(f, flag, (size_t)NT * 4)) || (r = up(tb, tBCellN, nc * 8)) || (r = up(sb, sBCellN, nc * 8)) ||
-      (r = up(dr, draws, nc * 8)) || (r = up(tp, tab.data(), tab.size() * 8)) || (r = up(err, nullptr, 4)))
+  if ((r = up_all({{&f, flag, (size_t)NT * 4}, {&tb, tBCellN, nc * 8}, {&sb, sBCellN, nc * 8}, {&dr, draws, nc * 8},
+                   {&tp, tab.data(), tab.size() * 8}, {&err, nullptr, 4}})))
     return r;
   DCHK(hipMemset(err.p, 0, 4));
   hipLaunchKernelGGL(k_react, dim3(nblk(numcell)), dim3(BT), 0, 0, (long long)numcell, NT, tb.as<long long>(),
                      sb.as<long long>(), dr.as<double>(), tp.as<double>(), f.as<int>(), err.as<int>());
   if ((r = read_err(err))) return r;
-  return down(flag, f, (size_t)NT * 4);
+  return copy_out({{flag, f.p, (size_t)NT * 4}}, 0);
 }
 
 extern "C" int mpcx_neighbour_list(int32_t NT, const double* box, double cutoff, double skinrad, const double* Xsol,
@@ -393,9 +407,7 @@ extern "C" int mpcx_neighbour_list(int32_t NT, const double* box, double cutoff,
   Buf x, y, z, sph;
   int r;
   double s[3] = {Xdim, Ydim, Zdim};
-  if ((r = up(x, Xsol, NT * 8ull)) || (r = up(y, Ysol, NT * 8ull)) || (r = up(z, Zsol, NT * 8ull)) ||
-      (r = up(sph, nullptr, 6 * 8)))
-    return r;
+  if ((r = up_all({{&x, Xsol, NT * 8ull}, {&y, Ysol, NT * 8ull}, {&z, Zsol, NT * 8ull}, {&sph, nullptr, 6 * 8}}))) return r;
   double sv[6] = {s[0], 0, s[1], 0, s[2], 0};   // layout (x[2*nd], y[2*nd], z[2*nd]) with nd = 1
   DCHK(hipMemcpy(sph.p, sv, sizeof sv, hipMemcpyHostToDevice));
   double full = cutoff + skinrad;
@@ -421,8 +433,7 @@ extern "C" int mpcx_inout_particle_list(int32_t NT, const double* box, double cu
   const int nd = numdims;
   std::vector<double> sv(6 * nd);
   for (int s = 0; s < 2 * nd; s++) { sv[s] = xdim[s]; sv[2 * nd + s] = ydim[s]; sv[4 * nd + s] = zdim[s]; }
-  if ((r = up(x, xsol, NT * 8ull)) || (r = up(y, ysol, NT * 8ull)) || (r = up(z, zsol, NT * 8ull)) ||
-      (r = up(sph, sv.data(), sv.size() * 8)))
+  if ((r = up_all({{&x, xsol, NT * 8ull}, {&y, ysol, NT * 8ull}, {&z, zsol, NT * 8ull}, {&sph, sv.data(), sv.size() * 8}})))
     return r;
   double fc = cutoffC + skinrad, fn = cutoffN + skinrad;
   std::vector<long long> in, out;
@@ -560,11 +571,10 @@ extern "C" int mpcx_distribute(int32_t NT, int32_t numdims, const int32_t* flag,
   for (int s = 0; s < 2 * nd; s++) { sv[s] = Xdim[s]; sv[2 * nd + s] = Ydim[s]; sv[4 * nd + s] = Zdim[s]; }
   Buf x, y, z, f, ol, il, sph, cnt, rank, ck, bucket, offb, err;
   int r;
-  if ((r = up(x, Xsol, NT * 8ull)) || (r = up(y, Ysol, NT * 8ull)) || (r = up(z, Zsol, NT * 8ull)) ||
-      (r = up(f, flag, NT * 4ull)) || (r = up(ol, outside_particle, no * 8)) || (r = up(il, inside_particle, ni * 8)) ||
-      (r = up(sph, sv.data(), sv.size() * 8)) || (r = up(cnt, nullptr, nk * 4)) || (r = up(rank, nullptr, nt * 4)) ||
-      (r = up(ck, nullptr, nt * 4)) || (r = up(bucket, nullptr, nt * 4)) || (r = up(offb, nullptr, (nk + 1) * 4)) ||
-      (r = up(err, nullptr, 4)))
+  if ((r = up_all({{&x, Xsol, NT * 8ull}, {&y, Ysol, NT * 8ull}, {&z, Zsol, NT * 8ull}, {&f, flag, NT * 4ull},
+                   {&ol, outside_particle, no * 8ull}, {&il, inside_particle, ni * 8ull}, {&sph, sv.data(), sv.size() * 8},
+                   {&cnt, nullptr, nk * 4ull}, {&rank, nullptr, nt * 4ull}, {&ck, nullptr, nt * 4ull},
+                   {&bucket, nullptr, nt * 4ull}, {&offb, nullptr, (nk + 1) * 4ull}, {&err, nullptr, 4}})))
     return r;
   DCHK(hipMemset(cnt.p, 0, nk * 4));
   DCHK(hipMemset(err.p, 0, 4));

@@ -13,6 +13,7 @@
 #include <vector>
 #include "mpcx_device.h"
 #include "mpcx_host.h"
+#include "mpcx_stage.h"
 #include "../../include/mpcx.h"
 
 namespace mpcx {
@@ -554,9 +555,7 @@ extern "C" int64_t mpcx_mlp_num_params(mpcx_mlp* e) { return e ? e->nparam : 0; 
 
 extern "C" int mpcx_mlp_get_params(mpcx_mlp* e, float* flat) {
   if (!e || !flat) return set_error(MPCX_E_ARG, "null argument");
-  MLCHK(hipStreamSynchronize(e->st));
-  MLCHK(hipMemcpy(flat, e->p, e->nparam * 4, hipMemcpyDeviceToHost));
-  return 0;
+  return mpcx::copy_out({{flat, e->p, (size_t)e->nparam * 4}}, e->st);
 }
 
 extern "C" int mpcx_mlp_set_params(mpcx_mlp* e, const float* flat) {
@@ -604,9 +603,7 @@ extern "C" int mpcx_mlp_forward(mpcx_mlp* e, int32_t rows, const float* x, float
     else launch(layer_forward<1, 1>);
     e->gemm_flops += 2ll * rows * N * e->dims[l];
   }
-  MLCHK(hipMemcpyAsync(y, e->Fy, (size_t)rows * e->n_out * 4, hipMemcpyDeviceToHost, e->st));
-  MLCHK(hipStreamSynchronize(e->st));
-  return 0;
+  return mpcx::copy_out({{y, e->Fy, (size_t)rows * e->n_out * 4}}, e->st);
 }
 
 // dataset rows, targets and output weights on the device
@@ -616,10 +613,8 @@ static int upload_data(mpcx_mlp* e, long long n, const float* x, const float* ta
   if ((rc = grow(e->st, e->X, e->x_n, n * e->n_in)) || (rc = grow(e->st, e->T, e->t_n, n * e->n_out)) ||
       (rc = grow(e->st, e->W, w_n, e->n_out)))
     return rc;
-  MLCHK(hipMemcpyAsync(e->X, x, (size_t)n * e->n_in * 4, hipMemcpyHostToDevice, e->st));
-  MLCHK(hipMemcpyAsync(e->T, target, (size_t)n * e->n_out * 4, hipMemcpyHostToDevice, e->st));
-  MLCHK(hipMemcpyAsync(e->W, wout, (size_t)e->n_out * 4, hipMemcpyHostToDevice, e->st));
-  return 0;
+  return mpcx::copy_in({mpcx::upload(e->X, x, (size_t)n * e->n_in * 4), mpcx::upload(e->T, target, (size_t)n * e->n_out * 4),
+                        mpcx::upload(e->W, wout, (size_t)e->n_out * 4)}, e->st);
 }
 static void launch_inputs(mpcx_mlp* e, long long n, int batch, long long steps, const int* idx) {
   const Act& a = e->H[0];

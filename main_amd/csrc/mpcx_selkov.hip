@@ -28,6 +28,7 @@
 #include <vector>
 #include "mpcx_device.h"
 #include "mpcx_host.h"
+#include "mpcx_stage.h"
 #include "mpcx_kernels.h"
 #include "../../include/mpcx.h"
 
@@ -1431,13 +1432,11 @@ extern "C" int mpcx_sk_get_state(mpcx_sk* e, double* x, double* y, double* z, do
   SkD& D = e->D;
   double* dst[9] = {x, y, z, vx, vy, vz, fx, fy, fz};
   double* src[9] = {D.x, D.y, D.z, D.vx, D.vy, D.vz, D.fx, D.fy, D.fz};
-  for (int a = 0; a < 9; a++)
-    if (dst[a]) SKCHK(hipMemcpy(dst[a], src[a], n * 8, hipMemcpyDeviceToHost));
-  if (flag) {
-    std::vector<int> f32(n);
-    SKCHK(hipMemcpy(f32.data(), D.flag, n * 4, hipMemcpyDeviceToHost));
-    for (size_t i = 0; i < n; i++) flag[i] = f32[i];
-  }
+  std::vector<mpcx::HostCopy> cp;
+  for (int a = 0; a < 9; a++) cp.push_back({dst[a], src[a], n * 8});
+  cp.push_back({flag, D.flag, n * 4, true});
+  const int rc = mpcx::copy_out(cp, e->st);
+  if (rc) return rc;
   if (dm) {
     std::vector<double> dim(24);
     SKCHK(hipMemcpy(dim.data(), D.dim, 24 * 8, hipMemcpyDeviceToHost));
