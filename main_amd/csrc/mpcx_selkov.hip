@@ -101,7 +101,13 @@ struct SkD {
 
 __device__ __forceinline__ int species(int f) { return f == 0 ? 0 : f == 1 ? 1 : f == 3 ? 2 : -1; }
 __device__ __forceinline__ bool active(int f) { return f == 0 || f == 1 || f == 3; }
-__device__ __forceinline__ double wrap(double x, double L) { return x - L * floor(x / L); }
+// x - L*floor(x/L) without the division for -L <= x < 2L: a correctly rounded
+// x/L lies in [-1,0), [0,1) or [1,2) exactly when x does, so the floor follows
+// by comparison and the subtraction is the same operation
+__device__ __forceinline__ double wrap(double x, double L) {
+  if (__builtin_expect(x < -L || x >= 2.0 * L, 0)) return x - L * floor(x / L);
+  return x < 0.0 ? x + L : (x >= L ? x - L : x);
+}
 
 // INT(FLOOR(X)+Box(1)*FLOOR(Y)+Box(1)*Box(2)*FLOOR(Z)+1) - 1
 __device__ __forceinline__ long long sk_cell0(const SkP& P, double x, double y, double z) {
@@ -189,10 +195,19 @@ __device__ __forceinline__ void sk_dimer_forces(const SkP& P, Dim2& d, const dou
 }
 
 // ------------------------------------------------------------- near engine
+constexpr int SK_R = 4;                // entries a thread holds in registers (sk_steps)
+constexpr int SK_A = SK_R * SK_T;      // entries of sk_steps
 struct SkShared {
-  double lx[SLCAP], ly[SLCAP], lz[SLCAP], lvx[SLCAP], lvy[SLCAP], lvz[SLCAP], lfx[SLCAP], lfy[SLCAP], lfz[SLCAP];
-  int lflag[SLCAP];
-  unsigned char lcflag[SLCAP];
+  union {
+    struct {   // general form: the near slots' state
+      double lx[SLCAP], ly[SLCAP], lz[SLCAP], lvx[SLCAP], lvy[SLCAP], lvz[SLCAP], lfx[SLCAP], lfy[SLCAP], lfz[SLCAP];
+      int lflag[SLCAP];
+    };
+    struct {   // sk_steps: each entry's C and N pair force and potential of the step, its near index
+      double fb[7][SK_A];
+      unsigned short eq[SK_A];
+    };
+  };
   double sd[12][2];
   double bond[3];
   double red[SK_W][8];
@@ -200,6 +215,7 @@ struct SkShared {
   int wsum[SK_W + 1];
   long long cursor, cstep;
   int nn;
+  double x0[3][2];   // spheres at the interval start (guard check)
   SkP P;
   SkD D;
 };
@@ -286,9 +302,9 @@ __device__ __attribute__((noinline)) void sk_begin_motion() {
   g_sk.bond[0] = d.bond[0]; g_sk.bond[1] = d.bond[1]; g_sk.bond[2] = d.bond[2];
 #pragma unroll
   for (int s = 0; s < 2; s++) {
-    double a = pbc_h(d.v[SX][s] - D.sc->x0[s], P.hbox[0], P.box[0]);
-    double b = pbc_h(d.v[SY][s] - D.sc->y0[s], P.hbox[1], P.box[1]);
-    double c = pbc_h(d.v[SZ][s] - D.sc->z0[s], P.hbox[2], P.box[2]);
+    double a = pbc_h(d.v[SX][s] - g_sk.x0[0][s], P.hbox[0], P.box[0]);
+    double b = pbc_h(d.v[SY][s] - g_sk.x0[1][s], P.hbox[1], P.box[1]);
+    double c = pbc_h(d.v[SZ][s] - g_sk.x0[2][s], P.hbox[2], P.box[2]);
     if (a * a + b * b + c * c > P.guard * P.guard) raise_error(&D.sc->err, ERR_NEAR_GUARD);
   }
 }
@@ -452,6 +468,353 @@ __device__ __forceinline__ void sk_first_motion(const SkP& P, const SkD& D, int 
   }
 }
 
+// The dimer's part of a step on wave 0 (every lane holds the dimer, lane 0
+// stores): the forces from the waves' sums in wave order (end), then the
+// motion that starts the next step and the guard check (begin).
+__device__ __forceinline__ void sk_dimer_step(const SkP& P, SkScalars* sc, bool end, bool begin, int lane) {
+  Dim2 d;
+#pragma unroll
+  for (int f = 0; f < 12; f++) { d.v[f][0] = g_sk.sd[f][0]; d.v[f][1] = g_sk.sd[f][1]; }
+  d.bond[0] = g_sk.bond[0]; d.bond[1] = g_sk.bond[1]; d.bond[2] = g_sk.bond[2];
+  if (end) {
+    double a = 0.0;
+    if (lane < 7) {
+      a = g_sk.red[0][lane];
+#pragma unroll
+      for (int w = 1; w < SK_W; w++) a = a + g_sk.red[w][lane];
+    }
+    double sum[7], tpot;
+#pragma unroll
+    for (int v = 0; v < 7; v++) sum[v] = lane_read_d(a, v);
+    sk_dimer_forces(P, d, sum, tpot, &sc->err);
+    if (lane == 0) sc->tpotential = tpot;
+  }
+  if (begin) {
+    sk_dimer_motion(P, d, &sc->err);
+    if (lane < 2) {
+      const double a = pbc_h((lane ? d.v[SX][1] : d.v[SX][0]) - g_sk.x0[0][lane], P.hbox[0], P.box[0]);
+      const double b = pbc_h((lane ? d.v[SY][1] : d.v[SY][0]) - g_sk.x0[1][lane], P.hbox[1], P.box[1]);
+      const double c = pbc_h((lane ? d.v[SZ][1] : d.v[SZ][0]) - g_sk.x0[2][lane], P.hbox[2], P.box[2]);
+      if (a * a + b * b + c * c > P.guard * P.guard) raise_error(&sc->err, ERR_NEAR_GUARD);
+    }
+  }
+  if (lane == 0) {
+#pragma unroll
+    for (int f = 0; f < 12; f++) { g_sk.sd[f][0] = d.v[f][0]; g_sk.sd[f][1] = d.v[f][1]; }
+    g_sk.bond[0] = d.bond[0]; g_sk.bond[1] = d.bond[1]; g_sk.bond[2] = d.bond[2];
+    if (begin) g_sk.cstep += 1;
+  }
+}
+
+// The wave's seven sums into g_sk.red[wv], bitwise those of wave_sum (lanes
+// 32, 16, 8, 4, 2, 1 apart): at the first three levels a lane keeps half of
+// its values and sends its partner the other half, so eight values take
+// 4 + 2 + 1 + 3 additions instead of eight times six.
+__device__ __forceinline__ double sk_keep(double x, double y, bool hi) { return hi ? y : x; }
+__device__ __forceinline__ void sk_reduce(const double (&a)[7], int wv, int lane) {
+  const bool b5 = lane & 32, b4 = lane & 16, b3 = lane & 8;
+  const double p0 = sk_keep(a[0], a[1], b5) + __shfl_xor(sk_keep(a[1], a[0], b5), 32, MPCX_WAVE);
+  const double p1 = sk_keep(a[2], a[3], b5) + __shfl_xor(sk_keep(a[3], a[2], b5), 32, MPCX_WAVE);
+  const double p2 = sk_keep(a[4], a[5], b5) + __shfl_xor(sk_keep(a[5], a[4], b5), 32, MPCX_WAVE);
+  const double p3 = sk_keep(a[6], 0.0, b5) + __shfl_xor(sk_keep(0.0, a[6], b5), 32, MPCX_WAVE);
+  const double q0 = sk_keep(p0, p1, b4) + __shfl_xor(sk_keep(p1, p0, b4), 16, MPCX_WAVE);
+  const double q1 = sk_keep(p2, p3, b4) + __shfl_xor(sk_keep(p3, p2, b4), 16, MPCX_WAVE);
+  double r = sk_keep(q0, q1, b3) + dpp_mov_d<DPP_ROW_ROR8>(sk_keep(q1, q0, b3));
+  r = r + dpp_xor4_d(r);
+  r = r + dpp_mov_d<DPP_QUAD_2301>(r);
+  r = r + dpp_mov_d<DPP_QUAD_1032>(r);
+  if ((lane & 7) == 0) g_sk.red[wv][(lane >> 5) + 2 * ((lane >> 4) & 1) + 4 * ((lane >> 3) & 1)] = r;
+}
+
+// The near set's MD steps with the particles that matter in registers.
+//
+// Most of the near set only might have come within a sphere's cutoff: a
+// particle farther from both cutoffs than its own flight of the launch plus
+// SK_QUIET of the guard flies freely while the spheres stay within that of
+// their start (checked every step), so it makes all its moves, the same
+// operations, at the start.  The others -- about 1,200 of 4,800 at 50^3 with
+// the reference input's physics -- are dealt evenly to the threads, whatever
+// lane the general form gives them, and stay in registers; their pair forces
+// go through LDS to the lane the general form sums them in, in its order
+// (entries ascending), so the sums are its sums bitwise.  In the general form
+// every step moved the whole set through LDS and L2 and one thread took the
+// dimer's step: 37 us a step at 50^3, 0.74 ms a launch.
+//
+// Device draws only: the parity stream's draws follow the order of the whole
+// set.  Returns false, with nothing done, when more than SK_A particles
+// matter; else `t_next` is the step after the last one done (before t1 + 1: the
+// spheres moved too far, the slots hold every particle at that step's start).
+constexpr double SK_QUIET = 0.1;   // of the guard: a sphere moves some 0.003 a launch at 50^3, a wider shell holds more particles
+__device__ __forceinline__ void sk_fly(const SkP& P, SkSlot& s, int moves) {
+  const bool on = active(s.flag);
+  const double dx = on ? s.vx * P.MDt : 0.0, dy = on ? s.vy * P.MDt : 0.0, dz = on ? s.vz * P.MDt : 0.0;
+  for (int k = 0; k < moves; k++) {
+    s.x = wrap(s.x + dx, P.box[0]);
+    s.y = wrap(s.y + dy, P.box[1]);
+    s.z = wrap(s.z + dz, P.box[2]);
+  }
+}
+__device__ __forceinline__ SkSlot sk_particle(const SkD& D, int p) {
+  SkSlot s;
+  s.x = D.x[p]; s.y = D.y[p]; s.z = D.z[p]; s.vx = D.vx[p]; s.vy = D.vy[p]; s.vz = D.vz[p];
+  s.fx = D.fx[p]; s.fy = D.fy[p]; s.fz = D.fz[p]; s.flag = D.flag[p];
+  return s;
+}
+__device__ __forceinline__ double sk_min_image2(const SkP& P, double x, double y, double z, int sph, double& d1, double& d2,
+                                                double& d3) {
+  d1 = x - g_sk.sd[SX][sph];
+  d2 = y - g_sk.sd[SY][sph];
+  d3 = z - g_sk.sd[SZ][sph];
+  if (__any(fabs(d1) > P.hbox[0] || fabs(d2) > P.hbox[1] || fabs(d3) > P.hbox[2])) {
+    d1 = pbc_h(d1, P.hbox[0], P.box[0]);
+    d2 = pbc_h(d2, P.hbox[1], P.box[1]);
+    d3 = pbc_h(d3, P.hbox[2], P.box[2]);
+  }
+  return d1 * d1 + d2 * d2 + d3 * d3;
+}
+// Before a launch of the near engine: which particles of its near set matter
+// (NF_MATTER in their census byte) and the slots of sk_steps -- a particle that
+// matters as it is, another one after the nmot motions of the launch.  The near
+// set lies scattered over the particle arrays (they are re-sorted every 10,000
+// steps), so its gather is the work of the whole chip: by the near engine's one
+// CU it took 0.2 ms, more than the MD steps.
+enum : unsigned char { NF_MATTER = 0x40 };
+__global__ __launch_bounds__(256) void sk_near_split(SkP P, SkD D, int nmot) {
+  __shared__ double sd[3][2];
+  if (threadIdx.x < 6) sd[threadIdx.x >> 1][threadIdx.x & 1] = D.dim[(SX + (threadIdx.x >> 1)) * 2 + (threadIdx.x & 1)];
+  __syncthreads();
+  const int nn = min(D.sc->near_num, D.near_cap);
+  for (int q = blockIdx.x * 256 + threadIdx.x; q < nn; q += gridDim.x * 256) {
+    SkSlot s = sk_particle(D, D.near_list[q]);
+    const double fly = sqrt((s.vx * s.vx + s.vy * s.vy) + s.vz * s.vz) * (P.MDt * (double)nmot) * (1.0 + 1e-9) +
+                       SK_QUIET * P.guard + 1e-9;
+    bool matter = s.fx != 0.0 || s.fy != 0.0 || s.fz != 0.0;
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      const double d1 = pbc_h(s.x - sd[0][i], P.hbox[0], P.box[0]), d2 = pbc_h(s.y - sd[1][i], P.hbox[1], P.box[1]),
+                   d3 = pbc_h(s.z - sd[2][i], P.hbox[2], P.box[2]);
+      const double o = (i == 0 ? P.cutC : P.cutN) + fly;
+      if (!(d1 * d1 + d2 * d2 + d3 * d3 > o * o)) matter = true;
+    }
+    if (matter) {
+      D.ns_vx[q] = s.vx; D.ns_vy[q] = s.vy; D.ns_vz[q] = s.vz;
+      D.ns_fx[q] = s.fx; D.ns_fy[q] = s.fy; D.ns_fz[q] = s.fz; D.ns_flag[q] = s.flag;
+    } else {
+      sk_fly(P, s, nmot);
+    }
+    D.ns_x[q] = s.x; D.ns_y[q] = s.y; D.ns_z[q] = s.z;
+    D.ns_cflag[q] = (unsigned char)(s.flag | (matter ? NF_MATTER : 0));
+  }
+}
+
+// One entry's step: forces with conversions, kick and, unless last, the next
+// motion; its forces into g_sk.fb[..][k] where they are or were not zero.
+// draw: some conversion probability lies strictly between 0 and 1 (a draw in
+// [0, 1) decides nothing else, and the draws are keyed, not consumed).
+__device__ __forceinline__ void sk_entry_step(const SkP& P, SkSlot& s, int p, int k, long long step, bool last, bool draw) {
+  const bool on = active(s.flag);
+  double n1, n2, n3, c1, c2, c3;
+  const double rN = sk_min_image2(P, s.x, s.y, s.z, 1, n1, n2, n3);
+  const double rC = sk_min_image2(P, s.x, s.y, s.z, 0, c1, c2, c3);
+  const bool inN = on && rN <= P.cutN2, inC = on && rC <= P.cutC2;
+  const bool had = s.fx != 0.0 || s.fy != 0.0 || s.fz != 0.0;
+  if (inN || inC || had) {
+    const double pfx = s.fx, pfy = s.fy, pfz = s.fz;
+    double pot = 0.0, nx = 0.0, ny = 0.0, nz = 0.0, cx = 0.0, cy = 0.0, cz = 0.0;
+    // one pair force for the lanes within one cutoff, whichever it is; a
+    // second only where a lane is within both
+    const bool firstN = inN;
+    if (inN || inC) {
+      const int b = firstN ? 1 : 0;
+      const double E_ = firstN ? g_sk.P.EN[s.flag] : g_sk.P.EC[s.flag];
+      double F, U;
+      lj_terms(firstN ? rN : rC, g_sk.P.R6[b], g_sk.P.R12[b], g_sk.P.r12R12[b], g_sk.P.r6R6[b], F, U);
+      const double EF = E_ * F;
+      const double fx = EF * (firstN ? n1 : c1), fy = EF * (firstN ? n2 : c2), fz = EF * (firstN ? n3 : c3);
+      pot = E_ * U;
+      if (firstN) { nx = fx; ny = fy; nz = fz; }
+      else { cx = fx; cy = fy; cz = fz; }
+      s.fx = fx; s.fy = fy; s.fz = fz;
+    } else {
+      s.fx = s.fy = s.fz = 0.0;
+    }
+    if (inN && inC) {   // the C sphere's force and potential stand (:123-234)
+      const double E_ = g_sk.P.EC[s.flag];
+      double F, U;
+      lj_terms(rC, P.R6[0], P.R12[0], P.r12R12[0], P.r6R6[0], F, U);
+      const double EF = E_ * F;
+      cx = EF * c1; cy = EF * c2; cz = EF * c3;
+      pot = E_ * U;
+      s.fx = cx; s.fy = cy; s.fz = cz;
+    }
+    if (inC && (s.flag == 0 || s.flag == 1)) {
+      const double pr = s.flag == 0 ? P.RPfg : P.RPgf;
+      bool conv = pr > 0.0;
+      if (draw) {
+        double u, v;
+        philox_uniform2(P.seed, 3, (unsigned long long)step, (unsigned long long)p, u, v);
+        conv = pr > u;
+      }
+      if (conv) s.flag = 1 - s.flag;
+    }
+    g_sk.fb[0][k] = cx; g_sk.fb[1][k] = cy; g_sk.fb[2][k] = cz;
+    g_sk.fb[3][k] = nx; g_sk.fb[4][k] = ny; g_sk.fb[5][k] = nz;
+    g_sk.fb[6][k] = pot;
+    if (on) {   // kick (:255-269) with the flag after the conversions
+      const double h = g_sk.P.hk[s.flag];
+      s.vx = s.vx + (pfx + s.fx) * h;
+      s.vy = s.vy + (pfy + s.fy) * h;
+      s.vz = s.vz + (pfz + s.fz) * h;
+    }
+  }
+  if (!last) {
+    if (on) {
+      const double h = g_sk.P.h2[s.flag];
+      s.x = (s.x + s.vx * P.MDt) + s.fx * h;
+      s.y = (s.y + s.vy * P.MDt) + s.fy * h;
+      s.z = (s.z + s.vz * P.MDt) + s.fz * h;
+    }
+    s.x = wrap(s.x, P.box[0]);
+    s.y = wrap(s.y, P.box[1]);
+    s.z = wrap(s.z, P.box[2]);
+  }
+}
+__device__ __forceinline__ bool sk_steps(const SkP& P, const SkD& D, int nn, int t0, int t1, int& t_next) {
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int E = sk_E(nn), qb = wv * 64 * E + lane;
+  const double margin = SK_QUIET * P.guard;
+  SkScalars* sc = D.sc;
+  // the lane's entries of the general form: those that matter (a bit each, from sk_near_split)
+  unsigned long long matter = 0ull;
+  for (int j = 0; j < E; j++) {
+    const int q = qb + j * 64;
+    if (q < nn && (D.ns_cflag[q] & NF_MATTER)) matter |= 1ull << j;
+  }
+  const int na = __popcll(matter);
+  const int incl = wave_incl_scan(na);
+  if (lane == 63) g_sk.wsum[wv] = incl;
+  sk_wave_scan();
+  const int NA = g_sk.wsum[SK_W];
+  if (NA > SK_A) return false;
+  const int base = g_sk.wsum[wv] + incl - na;   // the lane's entries: base .. base + na
+  {
+    int k = base;
+    for (unsigned long long m = matter; m; m &= m - 1ull) g_sk.eq[k++] = (unsigned short)(qb + 64 * (__ffsll(m) - 1));
+  }
+  for (int k = tid; k < NA; k += SK_T) {
+#pragma unroll
+    for (int v = 0; v < 7; v++) g_sk.fb[v][k] = 0.0;
+  }
+  const double sx0[2] = {g_sk.sd[SX][0], g_sk.sd[SX][1]}, sy0[2] = {g_sk.sd[SY][0], g_sk.sd[SY][1]},
+               sz0[2] = {g_sk.sd[SZ][0], g_sk.sd[SZ][1]};
+  __syncthreads();
+  SkSlot r[SK_R];
+  int p[SK_R];
+  unsigned cf = 0u;   // census flag of each entry, four bits
+#pragma unroll
+  for (int m = 0; m < SK_R; m++) {
+    const int k = m * SK_T + tid;
+    p[m] = -1;
+    if (k < NA) {
+      const int q = g_sk.eq[k];
+      p[m] = D.near_list[q];
+      r[m] = SkSlot{D.ns_x[q], D.ns_y[q], D.ns_z[q], D.ns_vx[q], D.ns_vy[q], D.ns_vz[q],
+                    D.ns_fx[q], D.ns_fy[q], D.ns_fz[q], D.ns_flag[q]};
+      cf |= (unsigned)r[m].flag << (4 * m);
+    } else {
+      r[m] = SkSlot{0, 0, 0, 0, 0, 0, 0, 0, 0, 2};
+    }
+  }
+#pragma unroll
+  for (int m = 0; m < SK_R; m++)
+    if (p[m] >= 0) sk_move(P, r[m]);
+  if (wv == 0) sk_dimer_step(P, sc, false, true, lane);
+  __syncthreads();
+  const bool draw = (P.RPfg > 0.0 && P.RPfg < 1.0) || (P.RPgf > 0.0 && P.RPgf < 1.0);
+  int t = t0;
+  while (t <= t1) {
+    // the spheres within the margin of their start (uniform)
+    bool near_start = true;
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      const double a = pbc_h(g_sk.sd[SX][i] - sx0[i], P.hbox[0], P.box[0]);
+      const double b = pbc_h(g_sk.sd[SY][i] - sy0[i], P.hbox[1], P.box[1]);
+      const double c = pbc_h(g_sk.sd[SZ][i] - sz0[i], P.hbox[2], P.box[2]);
+      near_start = near_start && a * a + b * b + c * c <= margin * margin;
+    }
+    if (!near_start) break;
+    const bool last = t == t1;
+    const long long step = g_sk.cstep;
+#pragma unroll
+    for (int m = 0; m < SK_R; m++)
+      if (p[m] >= 0) {
+        if (t == P.S) cf = (cf & ~(15u << (4 * m))) | ((unsigned)r[m].flag & 15u) << (4 * m);
+        sk_entry_step(P, r[m], p[m], m * SK_T + tid, step, last, draw);
+      }
+    __syncthreads();
+    double acc[7] = {0, 0, 0, 0, 0, 0, 0};
+    for (int k = base; k < base + na; k++) {
+#pragma unroll
+      for (int v = 0; v < 6; v++) acc[v] += g_sk.fb[v][k];
+      if (last) acc[6] += g_sk.fb[6][k];   // the potential is read after the launch only
+    }
+    sk_reduce(acc, wv, lane);
+    __syncthreads();
+    if (wv == 0) sk_dimer_step(P, sc, true, !last, lane);
+    __syncthreads();
+    t++;
+  }
+  t_next = t;
+  // write back: to the particle arrays when done, else to the slots of the
+  // general form at step t's start
+  const bool done = t > t1;
+  auto slot = [&](int q, const SkSlot& s, unsigned char census) {
+    D.ns_x[q] = s.x; D.ns_y[q] = s.y; D.ns_z[q] = s.z; D.ns_vx[q] = s.vx; D.ns_vy[q] = s.vy; D.ns_vz[q] = s.vz;
+    D.ns_fx[q] = s.fx; D.ns_fy[q] = s.fy; D.ns_fz[q] = s.fz; D.ns_flag[q] = s.flag;
+    D.ns_cflag[q] = census;
+  };
+#pragma unroll
+  for (int m = 0; m < SK_R; m++)
+    if (p[m] >= 0) {
+      const SkSlot& s = r[m];
+      const unsigned char census = (unsigned char)((cf >> (4 * m)) & 15u);
+      if (done) {
+        const int i = p[m];
+        D.x[i] = s.x; D.y[i] = s.y; D.z[i] = s.z; D.vx[i] = s.vx; D.vy[i] = s.vy; D.vz[i] = s.vz;
+        D.fx[i] = s.fx; D.fy[i] = s.fy; D.fz[i] = s.fz; D.flag[i] = s.flag;
+        const bool force = s.fx != 0.0 || s.fy != 0.0 || s.fz != 0.0;
+        D.cflag[i] = (unsigned char)(census | (force ? CF_FORCE : 0));
+      } else {
+        slot(g_sk.eq[m * SK_T + tid], s, census);
+      }
+    }
+  for (int j = 0; j < E; j++) {
+    const int q = qb + j * 64;
+    if (q >= nn || ((matter >> j) & 1ull)) continue;
+    const int i = D.near_list[q];
+    if (done) {
+      D.x[i] = D.ns_x[q]; D.y[i] = D.ns_y[q]; D.z[i] = D.ns_z[q];
+      D.cflag[i] = D.ns_cflag[q];
+    } else {
+      SkSlot s = sk_particle(D, i);
+      sk_fly(P, s, 1 + (t - t0));
+      slot(q, s, (unsigned char)s.flag);
+    }
+  }
+  if (!done) {
+    __threadfence_block();
+    __syncthreads();
+    for (int q = tid; q < min(nn, SLCAP); q += SK_T) {
+      g_sk.lx[q] = D.ns_x[q]; g_sk.ly[q] = D.ns_y[q]; g_sk.lz[q] = D.ns_z[q];
+      g_sk.lvx[q] = D.ns_vx[q]; g_sk.lvy[q] = D.ns_vy[q]; g_sk.lvz[q] = D.ns_vz[q];
+      g_sk.lfx[q] = D.ns_fx[q]; g_sk.lfy[q] = D.ns_fy[q]; g_sk.lfz[q] = D.ns_fz[q];
+      g_sk.lflag[q] = D.ns_flag[q];
+    }
+    __syncthreads();
+  }
+  return true;
+}
+
 // mode 0: steps 1..S of an interval (motion of step 1 first);
 // SM_STOP: steps 1..S-1, without the motion of step S (a sort comes first);
 // SM_RESUME: the motion and the step S.
@@ -467,6 +830,7 @@ __global__ __launch_bounds__(SK_T) void sk_near_engine(SkP P, SkD D, int mode) {
     for (int f = 0; f < 12; f++) { g_sk.sd[f][0] = D.dim[f * 2]; g_sk.sd[f][1] = D.dim[f * 2 + 1]; }
     if (!(mode & SM_RESUME))
       for (int s = 0; s < 2; s++) { sc->x0[s] = D.dim[SX * 2 + s]; sc->y0[s] = D.dim[SY * 2 + s]; sc->z0[s] = D.dim[SZ * 2 + s]; }
+    for (int s = 0; s < 2; s++) { g_sk.x0[0][s] = sc->x0[s]; g_sk.x0[1][s] = sc->y0[s]; g_sk.x0[2][s] = sc->z0[s]; }
   }
   __syncthreads();
   const int nn = g_sk.nn;
@@ -475,20 +839,25 @@ __global__ __launch_bounds__(SK_T) void sk_near_engine(SkP P, SkD D, int mode) {
     return;
   }
   unsigned long long T0 = __builtin_amdgcn_s_memrealtime();
-  sk_gather(D, nn);
-  __threadfence_block();
-  __syncthreads();
-  // motion of the launch's first step, solvent and dimer
-  sk_first_motion(P, D, nn);
-  if (tid == 0) {
-    g_sk.cstep += 1;
-    sk_begin_motion();
-  }
-  __threadfence_block();
-  __syncthreads();
   const int t0 = (mode & SM_RESUME) ? P.S : 1;
   const int t1 = (mode & SM_STOP) ? P.S - 1 : P.S;
-  for (int t = t0; t <= t1; t++) {
+  int t = t0;
+  const bool fast = P.rng_mode != 0 && t0 <= t1 && sk_steps(P, D, nn, t0, t1, t);
+  if (!fast) {
+    sk_gather(D, nn);
+    __threadfence_block();
+    __syncthreads();
+    // motion of the launch's first step, solvent and dimer
+    sk_first_motion(P, D, nn);
+    if (tid == 0) {
+      g_sk.cstep += 1;
+      sk_begin_motion();
+    }
+    __threadfence_block();
+    __syncthreads();
+  }
+  const bool slots = !fast || t <= t1;
+  for (; t <= t1; t++) {
     const bool last = (t == t1);
     if (P.rng_mode == 0) sk_count_draws();
     sk_step(last, t == P.S);
@@ -503,7 +872,7 @@ __global__ __launch_bounds__(SK_T) void sk_near_engine(SkP P, SkD D, int mode) {
     __threadfence_block();
     __syncthreads();
   }
-  sk_scatter(D, nn);
+  if (slots) sk_scatter(D, nn);
   if (tid == 0) {
     sc->cstep = g_sk.cstep;
     sc->cursor = g_sk.cursor;
@@ -1356,9 +1725,14 @@ extern "C" int mpcx_sk_run(mpcx_sk* e, int64_t ncoll, const double* draws, int64
     // device draws: the far particles stream and bin beside the near engine
     // (host draws: the shift is read at the draw cursor the near engine moves)
     const bool ov = e->overlap && P.rng_mode == 1 && !sort_due;
+    auto near = [&](int mode, int nmot) {   // the near engine's launch of nmot motions
+      if (P.rng_mode != 0) hipLaunchKernelGGL(sk_near_split, dim3(64), dim3(256), 0, st, P, D, nmot);
+      hipLaunchKernelGGL(sk_near_engine, dim3(1), dim3(SK_T), 0, st, P, D, mode);
+    };
     if (ov) SKCHK(hipEventRecord(e->fork, st));
     SKCHK(tmark(0, 0));
-    hipLaunchKernelGGL(sk_near_engine, dim3(1), dim3(SK_T), 0, st, P, D, sort_due ? SM_STOP : 0);
+    if (sort_due) near(SM_STOP, P.S - 1);
+    else near(0, P.S);
     SKCHK(tmark(0, 1));
     if (ov) {   // enqueued after the near engine, so that it is dispatched first
       SKCHK(hipStreamWaitEvent(e->st2, e->fork, 0));
@@ -1377,7 +1751,7 @@ extern "C" int mpcx_sk_run(mpcx_sk* e, int64_t ncoll, const double* draws, int64
       hipLaunchKernelGGL(sk_bulk, dim3(gN), dim3(256), 0, st, P, D, P.S - 1, 0, 0);
       sk_sort(e);
       sk_near_list(e);
-      hipLaunchKernelGGL(sk_near_engine, dim3(1), dim3(SK_T), 0, st, P, D, SM_RESUME);
+      near(SM_RESUME, 1);
       hipLaunchKernelGGL(sk_bulk, dim3(gN), dim3(256), 0, st, P, D, 1, 1, 0);
     } else {
       SKCHK(tmark(1, 0));
