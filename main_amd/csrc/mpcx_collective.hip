@@ -2022,6 +2022,80 @@ __device__ __forceinline__ int block_groups(const CoP& P, const CoD& D, GroupTab
 // slab 0: cell and rank for co_scatter; 1: the particle's slot in its cell's
 // slab written directly; 2: the same, and the cell must be listed late (the
 // particle was binned after the first collision pass).
+// Distance beyond the nearest list radius; 8 or more beyond every radius gives
+// 1e30 (the cap, 255 at 7.97) without a square root.
+__device__ __forceinline__ double list_distance(const CoP& P, double x, double y, double z, const double (*sph)[MAXSG]) {
+  double dmin = 1e30;
+  bool close = false;
+  for (int s = 0; s < 2 * P.nd; s++) {
+    double a = pbc_half(x - sph[0][s], P.box[0]);
+    double b = pbc_half(y - sph[1][s], P.box[1]);
+    double c = z - sph[2][s];
+    const double d2 = a * a + b * b + c * c, far = P.full[s >= P.nd] + 8.0;
+    close |= d2 < far * far;
+  }
+  if (__ballot(close))   // most waves lie far from every sphere: no square roots at all
+    for (int s = 0; s < 2 * P.nd; s++) {
+      double a = pbc_half(x - sph[0][s], P.box[0]);
+      double b = pbc_half(y - sph[1][s], P.box[1]);
+      double c = z - sph[2][s];
+      const double d2 = a * a + b * b + c * c, far = P.full[s >= P.nd] + 8.0;
+      if (d2 < far * far) dmin = fmin(dmin, sqrt(d2) - P.full[s >= P.nd]);
+    }
+  return dmin;
+}
+// The same for systems of many spheres (all lanes of the wave call it): only
+// the spheres that come within radius + 8 of the wave's bounding box are
+// looked at, found 64 at a time, a sphere a lane.  Sorted particles make small
+// boxes, so of the 200 spheres of a 100-dimer slab 4 or 5 remain; a scattered
+// wave's box keeps all of them, which only costs the test.  The box is kept in
+// FP32, widened by more than its rounding.  (co_bulk on that slab, 3.7 million
+// particles: 1.61 ms with every sphere looked at twice.)
+constexpr int CULL_MIN = 16;   // spheres from which the box pays (its six reductions cost about ten spheres)
+__device__ __forceinline__ double list_distance_culled(const CoP& P, bool valid, double x, double y, double z,
+                                                       const double (*sph)[MAXSG]) {
+  const int lane = threadIdx.x & 63;
+  const float big = 3e38f;
+  float c[3], h[3];
+  const double v[3] = {x, y, z};
+#pragma unroll
+  for (int a = 0; a < 3; a++) {
+    const float lo = wave_min_dpp_f(valid ? (float)v[a] : big), hi = -wave_min_dpp_f(valid ? -(float)v[a] : big);
+    c[a] = 0.5f * (lo + hi);
+    h[a] = 0.5f * (hi - lo) + 1e-3f + 1e-6f * (float)P.box[a];
+  }
+  double dmin = 1e30;
+  for (int s0 = 0; s0 < 2 * P.nd; s0 += 64) {
+    const int s = s0 + lane;
+    bool near = false;
+    if (s < 2 * P.nd) {
+      float d2 = 0.f;
+#pragma unroll
+      for (int a = 0; a < 3; a++) {
+        float d = fabsf(c[a] - (float)sph[a][s]);
+        if (a < 2) d = fminf(d, fabsf((float)P.box[a] - d));
+        d = fmaxf(d - h[a], 0.f);
+        d2 += d * d;
+      }
+      const float far = (float)P.full[s >= P.nd] + 8.01f;
+      near = d2 < far * far;
+    }
+    for (unsigned long long m = __ballot(near); m; m &= m - 1ull) {
+      const int q = s0 + __ffsll(m) - 1;
+      const double a = pbc_half(x - sph[0][q], P.box[0]);
+      const double b = pbc_half(y - sph[1][q], P.box[1]);
+      const double e = z - sph[2][q];
+      const double d2 = a * a + b * b + e * e, far = P.full[q >= P.nd] + 8.0;
+      if (__any(d2 < far * far)) {
+        if (d2 < far * far) dmin = fmin(dmin, sqrt(d2) - P.full[q >= P.nd]);
+      }
+    }
+  }
+  return dmin;
+}
+
+// CULL: systems of any number of dimers (else the few of a one-workgroup near engine)
+template <bool CULL>
 __device__ __forceinline__ void bin_particle(const CoP& P, const CoD& D, int i, bool valid, bool near,
                                              unsigned char st, double x, double y, double z, int f, double xs,
                                              double ys, double zs, const double (*sph)[MAXSG], int slab = 0) {
@@ -2048,6 +2122,8 @@ __device__ __forceinline__ void bin_particle(const CoP& P, const CoD& D, int i, 
     }
   }
   const int r = block_groups(P, D, G, t, ok, ck, cen, key);
+  const bool many = CULL && 2 * P.nd >= CULL_MIN;
+  double dmin = many ? list_distance_culled(P, valid, x, y, z, sph) : 0.0;
   if (valid) {
     if (ok && r >= BMAX) raise_error(&D.sc->err, ERR_BUCKET);
     D.cell_of[i] = t;
@@ -2056,25 +2132,7 @@ __device__ __forceinline__ void bin_particle(const CoP& P, const CoD& D, int i, 
       D.slab[(long long)t * BMAX + r] = i;
       if (slab == 2 && D.stamp[t] != D.epoch) raise_error(&D.sc->err, ERR_ZONE);
     }
-    // distance beyond the list radius; 8 or more beyond every radius gives the
-    // cap (255 at 7.97) without a sqrt
-    double dmin = 1e30;
-    bool close = false;
-    for (int s = 0; s < 2 * P.nd; s++) {
-      double a = pbc_half(x - sph[0][s], P.box[0]);
-      double b = pbc_half(y - sph[1][s], P.box[1]);
-      double c = z - sph[2][s];
-      const double d2 = a * a + b * b + c * c, far = P.full[s >= P.nd] + 8.0;
-      close |= d2 < far * far;
-    }
-    if (__ballot(close))   // most waves lie far from every sphere: no square roots at all
-      for (int s = 0; s < 2 * P.nd; s++) {
-        double a = pbc_half(x - sph[0][s], P.box[0]);
-        double b = pbc_half(y - sph[1][s], P.box[1]);
-        double c = z - sph[2][s];
-        const double d2 = a * a + b * b + c * c, far = P.full[s >= P.nd] + 8.0;
-        if (d2 < far * far) dmin = fmin(dmin, sqrt(d2) - P.full[s >= P.nd]);
-      }
+    if (!many) dmin = list_distance(P, x, y, z, sph);
     double qd = floor(fmax(dmin, 0.0) * 32.0 * (1.0 - 1e-12));
     if (st & ST_INSIDE) qd = 0.0;   // list members stay near until the next rebuild
     D.dq[i] = (unsigned char)fmin(qd, 255.0);
@@ -2137,7 +2195,7 @@ __device__ __forceinline__ void wall_defer(const CoD& D, bool wall, int i) {
 // in co_bin_rest, which also bins the near set once the near engine is done.
 // slab (FAR only): bin into the cells' slabs (first collision pass beside the
 // near engine); deferred particles then list their possible end cells late.
-template <bool FAR>
+template <bool FAR, bool CULL>
 __device__ __forceinline__ void bulk_body(const CoP& P, const CoD& D, int do_stream, int do_bin, long long first,
                                           long long end, long long step, int slab = 0) {
   const int nev = FAR ? 0 : min(D.sc->n_ev, MAXEV);
@@ -2216,18 +2274,18 @@ __device__ __forceinline__ void bulk_body(const CoP& P, const CoD& D, int do_str
     }
     if (FAR) wall_defer(D, wall, i);
     if (!do_bin) continue;
-    bin_particle(P, D, i, mine && !wall, near, st, x, y, z, f, xs, ys, zs, sph, slab);
+    bin_particle<CULL>(P, D, i, mine && !wall, near, st, x, y, z, f, xs, ys, zs, sph, slab);
   }
 }
 __global__ __launch_bounds__(256) void co_bulk(CoP P, CoD D, int do_stream, int do_bin) {
-  bulk_body<false>(P, D, do_stream, do_bin, (long long)blockIdx.x * blockDim.x, P.NT,
+  bulk_body<false, true>(P, D, do_stream, do_bin, (long long)blockIdx.x * blockDim.x, P.NT,
                    (long long)gridDim.x * blockDim.x);
 }
 // six waves per SIMD (at most 80 VGPRs, four of them spilled) where the
 // register count alone gave five: 0.376 -> 0.358 ms at 100^3 (seven waves
 // spilled sixteen and gained less)
 __global__ __launch_bounds__(256, 6) void co_far(CoP P, CoD D, int do_bin, int slab) {
-  bulk_body<true>(P, D, 1, do_bin, (long long)blockIdx.x * blockDim.x, P.NT, (long long)gridDim.x * blockDim.x,
+  bulk_body<true, false>(P, D, 1, do_bin, (long long)blockIdx.x * blockDim.x, P.NT, (long long)gridDim.x * blockDim.x,
                   slab);
 }
 // co_far's single flight covers the whole interval: the rebuild events
@@ -2271,7 +2329,7 @@ __global__ __launch_bounds__(256) void co_bin_rest(CoP P, CoD D, int do_bin, int
       st = D.status[i];
       if (!near) replay_events(P, D, i, x, y, z, f, ev, nev);
     }
-    if (do_bin) bin_particle(P, D, i, valid, near, st, x, y, z, f, xs, ys, zs, sph, slab ? 2 : 0);
+    if (do_bin) bin_particle<false>(P, D, i, valid, near, st, x, y, z, f, xs, ys, zs, sph, slab ? 2 : 0);
   }
   if (blockIdx.x == 0 && threadIdx.x == 0) check_flight(P, D);
 }
@@ -2280,7 +2338,7 @@ __global__ __launch_bounds__(256) void co_bulk_b(const CoP* Ps, const CoD* Ds, c
   const Tile t = tiles[blockIdx.x];
   const CoP P = Ps[t.r];
   const CoD D = Ds[t.r];
-  bulk_body<false>(P, D, do_stream, do_bin, t.begin, t.end, 256);
+  bulk_body<false, false>(P, D, do_stream, do_bin, t.begin, t.end, 256);
 }
 
 __device__ __forceinline__ void scatter_body(const CoD& D, long long first, long long end, long long step) {

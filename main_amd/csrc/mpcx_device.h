@@ -135,6 +135,19 @@ __device__ __forceinline__ double wave_max_dpp(double v) {
   v = fmax(v, dpp_mov_d<DPP_ROW_MIRROR>(v));
   return fmax(fmax(fmax(lane_read_d(v, 15), lane_read_d(v, 31)), lane_read_d(v, 47)), lane_read_d(v, 63));
 }
+// minimum over the wave (all 64 lanes active), wave-uniform; the maximum is -min(-v)
+template <int CTRL>
+__device__ __forceinline__ float dpp_mov_f(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
+}
+__device__ __forceinline__ float wave_min_dpp_f(float v) {
+  v = fminf(v, dpp_mov_f<DPP_QUAD_1032>(v));
+  v = fminf(v, dpp_mov_f<DPP_QUAD_2301>(v));
+  v = fminf(v, dpp_mov_f<DPP_ROW_HALF_MIRROR>(v));
+  v = fminf(v, dpp_mov_f<DPP_ROW_MIRROR>(v));
+  auto row = [&](int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l)); };
+  return fminf(fminf(row(15), row(31)), fminf(row(47), row(63)));
+}
 __device__ __forceinline__ int wave_sum_i(int v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, MPCX_WAVE);
