@@ -25,6 +25,7 @@
 #include <string>
 #include <vector>
 #include <algorithm>
+#include <type_traits>
 #include "mpcx_device.h"
 #include "mpcx_host.h"
 #include "mpcx_stage.h"
@@ -908,8 +909,8 @@ struct GeShared {
   int cstep, tc, tp, in_num, nev, rebuild;
   int qb, qe, ib, ie;
   unsigned ep;   // grid barriers passed in this launch
-  int rc[GE_GMAX];         // every workgroup's published count and max (ge_read_counts)
-  double rv[GE_GMAX];
+  int rc[2];               // counts before this workgroup and in all, and the max (ge_read_counts)
+  double rv;
   double vmax2, red[GE_W];
   unsigned long long tm[8];   // real-time ticks by phase (workgroup 0 reports them)
   unsigned touched[2][(MAXSG + 31) / 32];   // spheres this workgroup published, by step parity
@@ -927,10 +928,29 @@ __shared__ GeShared g_ge;
 #define GE_T0() const unsigned long long t0_ = __builtin_amdgcn_s_memrealtime()
 #define GE_T1(k) if (threadIdx.x == 0) g_ge.tm[k] += __builtin_amdgcn_s_memrealtime() - t0_
 
+// minimum over the wave, all 64 lanes active (on the VALU, as wave_sum_dpp)
 __device__ __forceinline__ int wave_min_i(int v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = min(v, __shfl_xor(v, o, MPCX_WAVE));
-  return v;
+  auto mv = [](int x, auto c) { return __builtin_amdgcn_update_dpp(0, x, decltype(c)::value, 0xf, 0xf, false); };
+  v = min(v, mv(v, std::integral_constant<int, DPP_QUAD_1032>{}));
+  v = min(v, mv(v, std::integral_constant<int, DPP_QUAD_2301>{}));
+  v = min(v, mv(v, std::integral_constant<int, DPP_ROW_HALF_MIRROR>{}));
+  v = min(v, mv(v, std::integral_constant<int, DPP_ROW_MIRROR>{}));
+  return min(min(wave_bcast(v, 15), wave_bcast(v, 31)), min(wave_bcast(v, 47), wave_bcast(v, 63)));
+}
+// Sums of four values over the wave, bitwise those of wave_sum (lanes 32, 16,
+// 8, 4, 2, 1 apart): at the first two levels a lane keeps half of its values
+// and sends its partner the other half; lanes 0, 32, 16 and 48 (and their
+// neighbours) end with values 0, 1, 2 and 3.
+__device__ __forceinline__ double wave_sum4(double a0, double a1, double a2, double a3, int lane) {
+  const bool b5 = lane & 32, b4 = lane & 16;
+  const double p0 = (b5 ? a1 : a0) + __shfl_xor(b5 ? a0 : a1, 32, MPCX_WAVE);
+  const double p1 = (b5 ? a3 : a2) + __shfl_xor(b5 ? a2 : a3, 32, MPCX_WAVE);
+  double r = (b4 ? p1 : p0) + __shfl_xor(b4 ? p0 : p1, 16, MPCX_WAVE);
+  r = r + dpp_mov_d<DPP_ROW_ROR8>(r);
+  r = r + dpp_xor4_d(r);
+  r = r + dpp_mov_d<DPP_QUAD_2301>(r);
+  r = r + dpp_mov_d<DPP_QUAD_1032>(r);
+  return r;
 }
 
 // Grid barrier of the G workgroups, run by wave 0 of each: every workgroup
@@ -1108,9 +1128,21 @@ __device__ __forceinline__ void ge_slot_store(const CoD& D, int k, double x, dou
     D.sl_flag[k] = fl; D.in_msd[k] = ms;
   }
 }
-// near slot q -> entry k of this workgroup
-__device__ __forceinline__ void ge_stage(const CoD& D, int k, int q, double ms) {
-  ge_slot_store(D, k, D.ns_x[q], D.ns_y[q], D.ns_z[q], D.ns_vx[q], D.ns_vy[q], D.ns_vz[q], D.ns_flag[q], ms);
+// near slots q -> entries k of this workgroup, four at a time
+__device__ __forceinline__ void ge_stage4(const CoD& D, const int (&k)[4], const int (&q)[4], const bool (&on)[4],
+                                          const double (&ms)[4]) {
+  double v[4][6];
+  int f[4];
+#pragma unroll
+  for (int u = 0; u < 4; u++)
+    if (on[u]) {
+      v[u][0] = D.ns_x[q[u]]; v[u][1] = D.ns_y[q[u]]; v[u][2] = D.ns_z[q[u]];
+      v[u][3] = D.ns_vx[q[u]]; v[u][4] = D.ns_vy[q[u]]; v[u][5] = D.ns_vz[q[u]];
+      f[u] = D.ns_flag[q[u]];
+    }
+#pragma unroll
+  for (int u = 0; u < 4; u++)
+    if (on[u]) ge_slot_store(D, k[u], v[u][0], v[u][1], v[u][2], v[u][3], v[u][4], v[u][5], f[u], ms[u]);
 }
 // this workgroup's entries -> their near slots
 __device__ __forceinline__ void ge_unstage(const CoD& D) {
@@ -1133,24 +1165,35 @@ __device__ __forceinline__ void ge_publish_count(const GeD& E, int c, double vm)
                        __HIP_MEMORY_SCOPE_AGENT);
   }
 }
-// (every thread together: one load per workgroup's words, one thread each,
-// where every thread loading all of them in turn waited on each)
+// (every thread together: wave 0 loads the words, two workgroups a lane, and
+// reduces them; every thread adding all of them up from LDS took 20 us a
+// rebuild at 128 workgroups)
 __device__ __forceinline__ void ge_read_counts(const GeD& E, int& before, int& total, double& vmax) {
-  const int G = (int)gridDim.x;
-  if ((int)threadIdx.x < G) {
-    g_ge.rc[threadIdx.x] = __hip_atomic_load(&E.sy->cnt[threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    g_ge.rv[threadIdx.x] = __longlong_as_double((long long)__hip_atomic_load(&E.sy->vmax2[threadIdx.x],
-                                                                              __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+  static_assert(GE_GMAX <= 128, "two workgroups a lane");
+  const int G = (int)gridDim.x, tid = (int)threadIdx.x;
+  if (tid < 64) {
+    int b = 0, t = 0;
+    double v = 0.0;
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      const int w = tid + 64 * u;
+      if (w >= G) continue;
+      const int c = __hip_atomic_load(&E.sy->cnt[w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      v = fmax(v, __longlong_as_double((long long)__hip_atomic_load(&E.sy->vmax2[w], __ATOMIC_RELAXED,
+                                                                     __HIP_MEMORY_SCOPE_AGENT)));
+      t += c;
+      if (w < (int)blockIdx.x) b += c;
+    }
+    b = wave_sum_i(b);
+    t = wave_sum_i(t);
+    v = wave_max(v);
+    if (tid == 0) { g_ge.rc[0] = b; g_ge.rc[1] = t; g_ge.rv = v; }
   }
   __syncthreads();
-  before = 0; total = 0; vmax = 0.0;
-  for (int w = 0; w < G; w++) {
-    const int c = g_ge.rc[w];
-    if (w < (int)blockIdx.x) before += c;
-    total += c;
-    vmax = fmax(vmax, g_ge.rv[w]);
-  }
-  __syncthreads();   // the words are read again by the next call
+  before = g_ge.rc[0];
+  total = g_ge.rc[1];
+  vmax = g_ge.rv;
+  __syncthreads();   // written again by the next call
 }
 
 // ordered compaction of this workgroup's near entries with pred(q) into
@@ -1162,9 +1205,20 @@ __device__ __forceinline__ void ge_compact_chunk(int base, Pred pred, Emit emit)
   const int E = (n + GE_T - 1) / GE_T;
   const int q0 = g_ge.qb + wv * 64 * E + lane;
   int cnt = 0;
-  for (int j = 0; j < E; j++) {
-    const int q = q0 + j * 64;
-    cnt += __popcll(__ballot(q < g_ge.qe && pred(q)));
+  unsigned long long mine = 0ull;   // the lane's own answers for the first 64 entries
+  constexpr int A = 8;   // answers whose loads are in flight together
+  for (int j0 = 0; j0 < E; j0 += A) {
+    bool in[A];
+#pragma unroll
+    for (int u = 0; u < A; u++) {
+      const int q = q0 + (j0 + u) * 64;
+      in[u] = j0 + u < E && q < g_ge.qe && pred(q);
+    }
+#pragma unroll
+    for (int u = 0; u < A; u++) {
+      if (j0 + u < 64) mine |= (unsigned long long)in[u] << (j0 + u);
+      cnt += __popcll(__ballot(in[u]));
+    }
   }
   if (lane == 0) g_ge.wsum[wv] = cnt;
   __syncthreads();
@@ -1176,13 +1230,23 @@ __device__ __forceinline__ void ge_compact_chunk(int base, Pred pred, Emit emit)
   __syncthreads();
   int b = base + g_ge.wsum[wv];
   const unsigned long long lt = lanes_below();
-  for (int j = 0; j < E; j++) {
-    const int q = q0 + j * 64;
-    const bool in = q < g_ge.qe && pred(q);
-    const unsigned long long bl = __ballot(in);
-    const int k = b + __popcll(bl & lt);
-    b += __popcll(bl);
-    if (in) emit(q, k);
+  // four entries a pass: emit loads them together, so that the L2 latency is
+  // paid once per pass
+  constexpr int B = 4;
+  for (int j0 = 0; j0 < E; j0 += B) {
+    int q[B], k[B];
+    bool in[B];
+#pragma unroll
+    for (int u = 0; u < B; u++) {
+      const int j = j0 + u;
+      q[u] = q0 + j * 64;
+      in[u] = j < 64 ? (mine >> j) & 1ull : (j < E && q[u] < g_ge.qe && pred(q[u]));
+      const unsigned long long bl = __ballot(in[u]);
+      k[u] = b + __popcll(bl & lt);
+      b += __popcll(bl);
+      if (j >= E || q[u] >= g_ge.qe) q[u] = -1;
+    }
+    emit(q, k, in);
   }
   __syncthreads();
 }
@@ -1201,18 +1265,37 @@ __device__ __attribute__((noinline)) void ge_rebuild(const CoP& P, const CoD& D,
   const double tc = (double)g_ge.tc;
   double vm = 0.0;
   int* err = &D.sc->err;
-  for (int q = g_ge.qb + threadIdx.x; q < g_ge.qe; q += GE_T) {
-    double x = D.ns_x[q], y = D.ns_y[q], z = D.ns_z[q], vx = D.ns_vx[q], vy = D.ns_vy[q], vz = D.ns_vz[q];
-    int f = D.ns_flag[q];
-    if (do_stream && !(D.ns_stat[q] & ST_INSIDE)) {
-      const int f0 = f;
-      bool b = stream_particle(x, y, z, vx, vy, vz, f, tc, P, D.react_box, err);
-      D.ns_x[q] = x; D.ns_y[q] = y; D.ns_z[q] = z;
-      if (b) { D.ns_vx[q] = vx; D.ns_vy[q] = vy; D.ns_vz[q] = vz; }
-      if (f != f0) D.ns_flag[q] = f;
+  int cnt = 0;   // members among the thread's entries
+  constexpr int B = 6;   // entries whose loads are in flight together
+  for (int q0 = g_ge.qb + threadIdx.x; q0 < g_ge.qe; q0 += B * GE_T) {
+    double x[B], y[B], z[B], vx[B], vy[B], vz[B];
+    int f[B];
+    unsigned char st[B];
+#pragma unroll
+    for (int u = 0; u < B; u++) {
+      const int q = q0 + u * GE_T;
+      if (q >= g_ge.qe) continue;
+      x[u] = D.ns_x[q]; y[u] = D.ns_y[q]; z[u] = D.ns_z[q]; vx[u] = D.ns_vx[q]; vy[u] = D.ns_vy[q]; vz[u] = D.ns_vz[q];
+      f[u] = D.ns_flag[q]; st[u] = D.ns_stat[q];
     }
-    vm = fmax(vm, (vx * vx + vy * vy) + vz * vz);
-    if (compact) E.memb_q[q] = ge_memberships(x, y, z, P, err);
+#pragma unroll
+    for (int u = 0; u < B; u++) {
+      const int q = q0 + u * GE_T;
+      if (q >= g_ge.qe) continue;
+      if (do_stream && !(st[u] & ST_INSIDE)) {
+        const int f0 = f[u];
+        bool b = stream_particle(x[u], y[u], z[u], vx[u], vy[u], vz[u], f[u], tc, P, D.react_box, err);
+        D.ns_x[q] = x[u]; D.ns_y[q] = y[u]; D.ns_z[q] = z[u];
+        if (b) { D.ns_vx[q] = vx[u]; D.ns_vy[q] = vy[u]; D.ns_vz[q] = vz[u]; }
+        if (f[u] != f0) D.ns_flag[q] = f[u];
+      }
+      vm = fmax(vm, (vx[u] * vx[u] + vy[u] * vy[u]) + vz[u] * vz[u]);
+      if (compact) {
+        const unsigned ids = ge_memberships(x[u], y[u], z[u], P, err);
+        E.memb_q[q] = ids;
+        cnt += ids != 0xffffffffu ? 1 : 0;
+      }
+    }
   }
   vm = wave_max(vm);
   if ((threadIdx.x & 63) == 0) g_ge.red[threadIdx.x >> 6] = vm;
@@ -1236,8 +1319,6 @@ __device__ __attribute__((noinline)) void ge_rebuild(const CoP& P, const CoD& D,
   }
   // members of this chunk, then their place in the system's inside list
   const auto member = [&](int q) { return E.memb_q[q] != 0xffffffffu; };
-  int cnt = 0;
-  for (int q = g_ge.qb + threadIdx.x; q < g_ge.qe; q += GE_T) cnt += member(q) ? 1 : 0;
   cnt = wave_sum_i(cnt);
   __syncthreads();
   if ((threadIdx.x & 63) == 0) g_ge.wsum[threadIdx.x >> 6] = cnt;
@@ -1265,15 +1346,26 @@ __device__ __attribute__((noinline)) void ge_rebuild(const CoP& P, const CoD& D,
     g_ge.tc = 0;
   }
   __syncthreads();
-  ge_compact_chunk(g_ge.ib, member, [&](int q, int k) {
-    if (k < E.in_cap) {
-      D.in_list[k] = q;
-      E.in_memb4[k] = E.memb_q[q];
-      if (k - g_ge.ib < GE_LCAP) g_ge.lmemb[k - g_ge.ib] = E.memb_q[q];
-      ge_stage(D, k, q, 0.0);
+  ge_compact_chunk(g_ge.ib, member, [&](const int (&q)[4], const int (&k)[4], const bool (&in)[4]) {
+    const double ms[4] = {0.0, 0.0, 0.0, 0.0};
+    unsigned mb[4];
+    bool on[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      on[u] = in[u] && k[u] < E.in_cap;
+      if (on[u]) mb[u] = E.memb_q[q[u]];
+    }
+    ge_stage4(D, k, q, on, ms);
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      if (on[u]) {
+        D.in_list[k[u]] = q[u];
+        E.in_memb4[k[u]] = mb[u];
+        if (k[u] - g_ge.ib < GE_LCAP) g_ge.lmemb[k[u] - g_ge.ib] = mb[u];
+      }
+      if (q[u] >= 0) D.ns_stat[q[u]] = in[u] ? ST_INSIDE : 0;
     }
   });
-  for (int q = g_ge.qb + threadIdx.x; q < g_ge.qe; q += GE_T) D.ns_stat[q] = member(q) ? ST_INSIDE : 0;
   if (threadIdx.x == 0) g_ge.ie = min(g_ge.ib + g_ge.wsum[GE_W], E.in_cap);
   __threadfence_block();
   __syncthreads();
@@ -1303,13 +1395,22 @@ __device__ __attribute__((noinline)) void ge_map_inside(const CoD& D, const GeD&
     g_ge.ib = min(before, E.in_cap);
   }
   __syncthreads();
-  ge_compact_chunk(g_ge.ib, ins, [&](int q, int k) {
-    if (k < E.in_cap) {
-      D.in_list[k] = q;
-      const int kl = k - g_ge.ib;
-      ge_stage(D, k, q, kl < GE_LCAP ? D.in_msd[k] : D.in_msd[k]);
-      if (kl < GE_LCAP) g_ge.lmemb[kl] = E.in_memb4[k];
+  ge_compact_chunk(g_ge.ib, ins, [&](const int (&q)[4], const int (&k)[4], const bool (&in)[4]) {
+    double ms[4];
+    unsigned mb[4];
+    bool on[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      on[u] = in[u] && k[u] < E.in_cap;
+      if (on[u]) { ms[u] = D.in_msd[k[u]]; mb[u] = E.in_memb4[k[u]]; }
     }
+    ge_stage4(D, k, q, on, ms);
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+      if (on[u]) {
+        D.in_list[k[u]] = q[u];
+        if (k[u] - g_ge.ib < GE_LCAP) g_ge.lmemb[k[u] - g_ge.ib] = mb[u];
+      }
   });
   if (threadIdx.x == 0) g_ge.ie = min(g_ge.ib + g_ge.wsum[GE_W], E.in_cap);
   __syncthreads();
@@ -1410,10 +1511,10 @@ __device__ __attribute__((noinline)) double ge_particles(const CoP& P, const CoD
         for (int m = 0; m < 4; m++)
           if (m == ptr) { c0 = fx[m]; c1 = fy[m]; c2 = fz[m]; c3 = pot[m]; }
       }
-      c0 = wave_sum(c0); c1 = wave_sum(c1); c2 = wave_sum(c2); c3 = wave_sum(c3);
-      if (lane == 0) {
-        double* a = &g_ge.wacc[wv][4 * smin];
-        a[0] = a[0] + c0; a[1] = a[1] + c1; a[2] = a[2] + c2; a[3] = a[3] + c3;
+      const double r = wave_sum4(c0, c1, c2, c3, lane);
+      if ((lane & 15) == 0) {
+        double* a = &g_ge.wacc[wv][4 * smin + (lane >> 5) + 2 * ((lane >> 4) & 1)];
+        *a = *a + r;
       }
       if (mine) ptr++;
     }
@@ -1668,11 +1769,27 @@ __global__ __launch_bounds__(GE_T) void co_ge_engine(CoP P, CoD D, GeD E, int ns
   }
   __syncthreads();
   // near particles of this chunk into their slots
-  for (int q = g_ge.qb + tid; q < g_ge.qe; q += GE_T) {
-    const int p = D.near_list[q];
-    D.ns_x[q] = D.x[p]; D.ns_y[q] = D.y[p]; D.ns_z[q] = D.z[p];
-    D.ns_vx[q] = D.vx[p]; D.ns_vy[q] = D.vy[p]; D.ns_vz[q] = D.vz[p];
-    D.ns_flag[q] = D.flag[p]; D.ns_stat[q] = D.status[p];
+  for (int q0 = g_ge.qb + tid; q0 < g_ge.qe; q0 += 4 * GE_T) {
+    int p[4], f[4];
+    double v[4][6];
+    unsigned char st[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) p[u] = q0 + u * GE_T < g_ge.qe ? D.near_list[q0 + u * GE_T] : -1;
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+      if (p[u] >= 0) {
+        v[u][0] = D.x[p[u]]; v[u][1] = D.y[p[u]]; v[u][2] = D.z[p[u]];
+        v[u][3] = D.vx[p[u]]; v[u][4] = D.vy[p[u]]; v[u][5] = D.vz[p[u]];
+        f[u] = D.flag[p[u]]; st[u] = D.status[p[u]];
+      }
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+      if (p[u] >= 0) {
+        const int q = q0 + u * GE_T;
+        D.ns_x[q] = v[u][0]; D.ns_y[q] = v[u][1]; D.ns_z[q] = v[u][2];
+        D.ns_vx[q] = v[u][3]; D.ns_vy[q] = v[u][4]; D.ns_vz[q] = v[u][5];
+        D.ns_flag[q] = f[u]; D.ns_stat[q] = st[u];
+      }
   }
   __threadfence_block();
   __syncthreads();
