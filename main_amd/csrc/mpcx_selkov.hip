@@ -1759,14 +1759,15 @@ extern "C" int mpcx_sk_run(mpcx_sk* e, int64_t ncoll, const double* draws, int64
       SKCHK(tmark(1, 1));
     }
     hipLaunchKernelGGL(sk_affected, dim3(1), dim3(256), 0, st, P, D);
-    launch_scan(st, D.unaff, V, D.partial, D.uoff);
+    if (P.rng_mode == 0) launch_scan(st, D.unaff, V, D.partial, D.uoff);   // the parity stream's draw slots
     launch_scan(st, D.cnt, V, D.partial, D.off);
     hipLaunchKernelGGL(sk_scatter_cells, dim3(gN), dim3(256), 0, st, P, D);
     SKCHK(tmark(2, 0));
     hipLaunchKernelGGL(sk_collide, dim3((unsigned)((V + CT - 1) / CT)), dim3(CT), 0, st, P, D);
     SKCHK(tmark(2, 1));
-    hipLaunchKernelGGL(sk_rotate_begin, dim3(grid_for(e->nwords + 2, 256, 2048)), dim3(256), 0, st, P, D,
-                       ov ? 0LL : (long long)(e->nwords + 2));
+    if (!ov)   // (with the overlap sk_rotate clears as it goes, and device draws have no cursor)
+      hipLaunchKernelGGL(sk_rotate_begin, dim3(grid_for(e->nwords + 2, 256, 2048)), dim3(256), 0, st, P, D,
+                         (long long)(e->nwords + 2));
     SKCHK(tmark(3, 0));
     hipLaunchKernelGGL(sk_rotate, dim3(gN), dim3(256), 0, st, P, D, ov ? 1 : 0);
     SKCHK(tmark(3, 1));
