@@ -39,9 +39,10 @@ int mpcx_device_count(void);
 /* hipDeviceSynchronize on the current device */
 int mpcx_device_synchronize(void);
 /* No counterpart in the reference: destroys every engine, batch and network
- * still live (batches first) and drains the device, so no stream, event,
- * graph or buffer outlives the HIP runtime at process exit.  Handles are
- * invalid afterwards.  The Python front end calls it at interpreter exit. */
+ * still live (batches first), drains the device and gives back the pinned
+ * copy ring and the drop-ins' device blocks, so no stream, event, graph or
+ * buffer outlives the HIP runtime at process exit.  Handles are invalid
+ * afterwards.  The Python front end calls it at interpreter exit. */
 int mpcx_shutdown(void);
 /* Measurement aid with no counterpart in the reference: copies nbytes between
  * two device buffers reps times (after one warm-up copy) and returns the mean

@@ -1,12 +1,12 @@
 // Collective engine: the MD + MPC time loop of collective_code on one MI355X.
 //
 // Work split per collision interval (MPCtstep MD steps + one collision):
-//  * near engine (one persistent 1024-thread workgroup per system): the
+//  * near engine (one persistent 768-thread workgroup per system): the
 //    particles that can enter a neighbour list during the interval ("near"
 //    set) are advanced exactly like evolve_mod.f95:6-732 -- inside particles
-//    live in registers across all MD steps, the dimer lives in LDS and is
-//    integrated by thread 0 (RATTLE), neighbour lists are rebuilt by ordered
-//    block-wide compaction of the near set.
+//    live in LDS across the MD steps between rebuilds, each dimer lives in LDS
+//    and is integrated by one wave (RATTLE), neighbour lists are rebuilt by
+//    ordered block-wide compaction of the near set.
 //  * bulk kernels over all particles: the "far" particles are only ever
 //    touched by the lazy streaming of evolve_mod.f95:467-529; the rebuild
 //    schedule recorded by the near engine is replayed in registers in one
@@ -36,7 +36,7 @@
 
 namespace mpcx {
 
-constexpr int NE_T = 768;    // near-engine threads (one workgroup, 256 VGPRs per lane)
+constexpr int NE_T = 768;    // near-engine threads (one workgroup, 168 VGPRs per lane)
 constexpr int NE_CAP = 16384;  // inside-list capacity of the near engine
 constexpr int MAXD = 4;      // dimers one near-engine workgroup handles (a cluster)
 constexpr int MAXS = 2 * MAXD;
@@ -280,9 +280,10 @@ __device__ __forceinline__ double wrap_periodic_any(double X, double L) {
   return wrap_periodic(X, L);
 }
 
-// ------------------------------------------------------------- dimer (thread 0)
-// The dimer state of one system, held in registers while thread 0 integrates
-// it (all indices are compile-time after unrolling).  Sphere s = k + i*ND.
+// ------------------------------------------------------------- dimer
+// The dimer state of one system, held in registers while it is integrated (by
+// the lanes of one wave, or by one thread in the global engine; all indices
+// are compile-time after unrolling).  Sphere s = k + i*ND.
 template <int ND>
 struct Dimer {
   double v[12][2 * ND];
@@ -1250,7 +1251,6 @@ __device__ __forceinline__ void ge_compact_chunk(int base, Pred pred, Emit emit)
   }
   __syncthreads();
 }
-__device__ __forceinline__ int ge_count_chunk_pred_total() { return g_ge.wsum[GE_W]; }
 
 // Rebuild over this workgroup's chunk: lazy streaming of its near particles
 // outside the lists (when do_stream), memberships, then the ordered
@@ -1523,7 +1523,7 @@ __device__ __attribute__((noinline)) double ge_particles(const CoP& P, const CoD
 }
 
 // thread s < 2 nd of workgroup 0: forces on sphere s (evolve_mod.f95:605-636,
-// the order of dimer_forces_and_rattle_v)
+// the order of dimer_forces_and_rattle_v_wave)
 __device__ __forceinline__ void ge_sphere_force(const CoP& P, int s) {
   const int nd = P.nd, k = s < nd ? s : s - nd, i = s < nd ? 0 : 1;
   double fw, wp;
@@ -1552,7 +1552,7 @@ __device__ __forceinline__ void ge_sphere_force(const CoP& P, int s) {
   g_ge.tpp[s] = tp;
 }
 // thread k < nd of workgroup 0: one dimer through rattle_positions / the
-// velocity RATTLE of dimer_forces_and_rattle_v (the same arithmetic)
+// velocity RATTLE of dimer_forces_and_rattle_v_wave (the same arithmetic)
 __device__ __forceinline__ void ge_dimer_load(Dimer<1>& d, int k, int nd) {
   for (int f = 0; f < 12; f++) { d.v[f][0] = g_ge.dim[f][k]; d.v[f][1] = g_ge.dim[f][k + nd]; }
 }
@@ -2167,7 +2167,7 @@ __device__ __forceinline__ double list_distance(const CoP& P, double x, double y
 // boxes, so of the 200 spheres of a 100-dimer slab 4 or 5 remain; a scattered
 // wave's box keeps all of them, which only costs the test.  The box is kept in
 // FP32, widened by more than its rounding.  (co_bulk on that slab, 3.7 million
-// particles: 1.61 ms with every sphere looked at twice.)
+// particles: 1.61 ms with every sphere looked at twice, 0.33 ms so.)
 constexpr int CULL_MIN = 16;   // spheres from which the box pays (its six reductions cost about ten spheres)
 __device__ __forceinline__ double list_distance_culled(const CoP& P, bool valid, double x, double y, double z,
                                                        const double (*sph)[MAXSG]) {
@@ -3890,7 +3890,7 @@ __global__ __launch_bounds__(256) void co_restart_sums(CoP P, CoD D, GeD E, int 
 }
 
 // dimer forces and potential from the totals (the force part of
-// dimer_forces_and_rattle_v, velocities untouched)
+// dimer_forces_and_rattle_v_wave, velocities untouched)
 __global__ __launch_bounds__(256) void co_restart_dimers(CoP P, CoD D, const double* sums) {
   __shared__ double tp[MAXSG];
   const int nd = P.nd, s = threadIdx.x;

@@ -172,14 +172,6 @@ __device__ __forceinline__ unsigned long long wave_incl_scan64(unsigned long lon
   }
   return v;
 }
-// rank of this lane among lanes (of lower id) whose predicate holds
-__device__ __forceinline__ int wave_rank(bool pred, unsigned long long& mask) {
-  mask = __ballot(pred);
-  int lane = threadIdx.x & (MPCX_WAVE - 1);
-  unsigned long long lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-  return __popcll(mask & lt);
-}
-
 // Block exclusive scan of a 64-bit value over blockDim.x threads (fixed order,
 // so results are deterministic).  scratch: >= blockDim.x/64 + 1 entries.
 __device__ __forceinline__ unsigned long long block_excl_scan64(unsigned long long v,
