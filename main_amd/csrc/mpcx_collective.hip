@@ -2167,7 +2167,7 @@ __device__ __forceinline__ double list_distance(const CoP& P, double x, double y
 // boxes, so of the 200 spheres of a 100-dimer slab 4 or 5 remain; a scattered
 // wave's box keeps all of them, which only costs the test.  The box is kept in
 // FP32, widened by more than its rounding.  (co_bulk on that slab, 3.7 million
-// particles: 1.61 ms with every sphere looked at twice, 0.33 ms so.)
+// particles: 1.61 ms with every sphere looked at twice, 0.21 ms so.)
 constexpr int CULL_MIN = 16;   // spheres from which the box pays (its six reductions cost about ten spheres)
 __device__ __forceinline__ double list_distance_culled(const CoP& P, bool valid, double x, double y, double z,
                                                        const double (*sph)[MAXSG]) {
