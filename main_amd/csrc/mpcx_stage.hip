@@ -49,10 +49,16 @@ void ring_release() {
   }
   g_ring.dev = -1;
 }
-// the ring on the current device, or false (the caller copies plainly)
-bool ring_ready() {
-  int dev = -1;
+// the ring on the current device, or false (the caller copies plainly): no
+// pinned memory to be had, or a stream of another device, whose work the
+// ring's events cannot mark
+bool ring_ready(hipStream_t st) {
+  int dev = -1, sdev = -1;
   if (hipGetDevice(&dev) != hipSuccess) return false;
+  if (st && (hipStreamGetDevice(st, &sdev) != hipSuccess || sdev != dev)) {
+    (void)hipGetLastError();
+    return false;
+  }
   if (g_ring.pin && g_ring.dev == dev) return true;
   ring_release();
   if (hipHostMalloc((void**)&g_ring.pin, SLOT * NSLOT, hipHostMallocDefault) != hipSuccess) {
@@ -233,7 +239,7 @@ int copy(const std::vector<HostCopy>& v, bool out, hipStream_t st) {
     if (c.host) total += c.bytes;
   if (total >= MIN_STAGED) {
     std::unique_lock<std::mutex> l(g_ring.mu, std::try_to_lock);
-    if (l.owns_lock() && ring_ready()) return staged(v, out, st, total);
+    if (l.owns_lock() && ring_ready(st)) return staged(v, out, st, total);
   }
   return plain(v, out, st);
 }
