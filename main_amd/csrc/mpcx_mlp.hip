@@ -244,6 +244,7 @@ struct GradLayer {
   __bf16 *w, *wt;           // BF16 copies of the weights
   long long woff, boff;     // in the flat parameters
   int N, K, ldw, ldwt, nt;  // dims, leading dimensions, tiles along K
+  int ldh;                  // leading dimension of Ht
   int blk0, bias0;          // first workgroup of its tiles and of its bias
 };
 struct GradArgs {
@@ -276,7 +277,7 @@ __global__ __launch_bounds__(256) void layer_grads(GradArgs G, int rows, int ldt
   if (!my_tile<1, 1>((L.N + 15) / 16, L.nt, (int)blockIdx.x - L.blk0, m0, n0)) return;
   const int gn = TILE_COL(0), gm = TILE_ROW(0);
   f32x4 acc[1][1];
-  tile_product<1, 1>(L.dZt, ldt, L.Ht, ldt, (rows + PAD - 1) / PAD * PAD, m0, n0, acc);
+  tile_product<1, 1>(L.dZt, ldt, L.Ht, L.ldh, (rows + PAD - 1) / PAD * PAD, m0, n0, acc);
   if (gn >= L.K) return;
   float w[4];
 #pragma unroll
@@ -304,9 +305,9 @@ __global__ void weights_bf16(int N, int K, const float* __restrict__ W, __bf16* 
   }
 }
 
-// The input rows of every batch of an epoch, BF16 by row and transposed, zeros
+// The input rows of `steps` batches in a row, BF16 by row and transposed, zeros
 // to the batches' padded sizes: row r of batch s is row idx[s*batch + r] of X
-// (idx null: row s*batch + r).
+// (idx null: row s*batch + r), of the n rows left.
 __global__ void input_rows(int n, int batch, int steps, int cols, const float* __restrict__ X, const int* __restrict__ idx,
                            __bf16* __restrict__ hb, int ldb, __bf16* __restrict__ ht, int ldt, int cols_p) {
   const long long per = (long long)ldt * cols;
@@ -347,7 +348,7 @@ struct mpcx_mlp {
   float *Fx = nullptr, *Fy = nullptr;
   // training buffers (cap rows a batch)
   int cap = 0;
-  std::vector<Act> H, dZ;             // H[0]: the input rows of a whole epoch's batches
+  std::vector<Act> H, dZ;             // H[0]: the input rows of several batches (its ldt: the call's padded batch)
   long long in_rows = 0;              // rows H[0] holds
   double *part = nullptr, *loss = nullptr;
   long long part_n = 0, loss_n = 0;
@@ -400,8 +401,18 @@ static int make_act(hipStream_t st, Act& a, long long rows, int ldt, int cols) {
   return 0;
 }
 
-// training buffers for batches of `batch` rows, `steps` of them an epoch
-static int train_buffers(mpcx_mlp* e, int batch, long long steps) {
+// Training buffers for batches of `batch` rows, `steps` of them an epoch; held:
+// the batches whose input rows and loss shares are on the device together.
+// These are laid out for the call's own batch, and an epoch of more than
+// HELD_BYTES of them is taken in parts: with the largest batch seen as their
+// stride, or a whole epoch held, the memory of a small batch's epoch was the
+// product of two sizes that need not meet (320 GB for 50,000 rows one at a time
+// after a gradient of all of them).
+constexpr long long HELD_BYTES = 64ll << 20;
+static long long part_stride(const mpcx_mlp* e) {
+  return (long long)(e->H[0].ldt / 16) * ((e->n_out + 15) / 16) + 4;
+}
+static int train_buffers(mpcx_mlp* e, int batch, long long steps, long long& held) {
   const int L = (int)e->dims.size(), R = up32(batch);
   int rc;
   if (batch > e->cap) {
@@ -416,30 +427,27 @@ static int train_buffers(mpcx_mlp* e, int batch, long long steps) {
     }
     e->cap = batch;
   }
-  const int ldt = up32(e->cap);
-  if (ldt * steps > e->in_rows) {
-    release_act(e->H[0]);
-    e->H[0] = Act{};
-    e->H[0].cols = e->n_in; e->H[0].ldb = up32(e->n_in); e->H[0].ldt = ldt;
+  Act& in = e->H[0];
+  in.cols = e->n_in; in.ldb = up32(e->n_in); in.ldt = R;
+  held = std::max(1ll, std::min(steps, HELD_BYTES / ((long long)R * in.ldb * 4 + part_stride(e) * 8)));
+  if (R * held > e->in_rows) {
+    release_act(in);
     e->in_rows = 0;
-    if ((rc = zeroed(e->st, e->H[0].b, (size_t)ldt * steps * e->H[0].ldb)) ||
-        (rc = zeroed(e->st, e->H[0].t, (size_t)ldt * steps * e->H[0].ldb)))
+    if ((rc = zeroed(e->st, in.b, (size_t)R * held * in.ldb)) || (rc = zeroed(e->st, in.t, (size_t)R * held * in.ldb)))
       return rc;
-    e->in_rows = ldt * steps;
+    e->in_rows = R * held;
   }
-  const long long tiles = (long long)(ldt / 16) * ((e->n_out + 15) / 16) + 4;
-  if ((rc = grow(e->st, e->part, e->part_n, tiles * steps))) return rc;
-  return 0;
+  return grow(e->st, e->part, e->part_n, part_stride(e) * held);
 }
 
-// one training step's forward and backward on batch s of the epoch's input
+// one training step's forward and backward on batch s of the held input
 // rows; the loss shares into the step's part, the gradients applied (a.on) or into g
 static void train_step(mpcx_mlp* e, int rows, long long s, const float* T, const int* idx, const float* wout, Adam a) {
   const int L = (int)e->dims.size(), ldt = up32(e->cap), Rp = up32(rows), mt = Rp / 16;
   hipStream_t st = e->st;
-  const __bf16* in = e->H[0].b + (size_t)s * ldt * e->H[0].ldb;
-  const __bf16* int_ = e->H[0].t + (size_t)s * ldt * e->H[0].ldb;
-  const long long tiles = (long long)(ldt / 16) * ((e->n_out + 15) / 16) + 4;
+  const Act& X = e->H[0];
+  const __bf16* in = X.b + (size_t)s * X.ldt * X.ldb;
+  const __bf16* int_ = X.t + (size_t)s * X.ldt * X.ldb;
   for (int l = 0; l + 1 < L; l++) {
     const int K = up32(e->dims[l]), N = e->dims[l + 1], nt = (N + 15) / 16;
     const unsigned grid = (unsigned)((mt * nt + 3) / 4);
@@ -449,7 +457,7 @@ static void train_step(mpcx_mlp* e, int rows, long long s, const float* T, const
                          (const __bf16*)e->w[l], K, (const float*)(e->p + e->boff[l]), 1, e->H[l + 1]);
     else
       hipLaunchKernelGGL(output_loss, dim3(grid), dim3(256), 0, st, rows, mt, nt, K, A, K, (const __bf16*)e->w[l], K,
-                         (const float*)(e->p + e->boff[l]), T, idx, wout, e->dZ[l + 1], e->part + s * tiles);
+                         (const float*)(e->p + e->boff[l]), T, idx, wout, e->dZ[l + 1], e->part + s * part_stride(e));
     e->gemm_flops += 2ll * rows * N * e->dims[l];
   }
   for (int l = L - 2; l >= 1; l--) {
@@ -465,7 +473,7 @@ static void train_step(mpcx_mlp* e, int rows, long long s, const float* T, const
       GradLayer& q = G.l[G.n++];
       const int N = e->dims[l + 1], K = e->dims[l];
       q = GradLayer{e->dZ[l + 1].t, l ? e->H[l].t : int_, e->dZ[l + 1].f, e->w[l], e->wt[l], e->woff[l], e->boff[l],
-                    N, K, up32(K), up32(N), (K + 15) / 16, blk, 0};
+                    N, K, up32(K), up32(N), (K + 15) / 16, l ? ldt : X.ldt, blk, 0};
       blk += ((N + 15) / 16 * q.nt + 3) / 4;
       q.bias0 = blk;
       blk += (N + 255) / 256;
@@ -621,9 +629,10 @@ static void launch_inputs(mpcx_mlp* e, long long n, int batch, long long steps, 
   hipLaunchKernelGGL(input_rows, dim3(blocks_for((long long)a.ldt * a.cols * steps)), dim3(256), 0, e->st, (int)n, batch,
                      (int)steps, a.cols, (const float*)e->X, idx, a.b, a.ldb, a.t, a.ldt, a.ldb);
 }
-static void launch_loss(mpcx_mlp* e, int tiles, long long steps, double* out) {
-  const long long stride = (long long)(up32(e->cap) / 16) * ((e->n_out + 15) / 16) + 4;
-  hipLaunchKernelGGL(loss_sums, dim3((unsigned)steps), dim3(64), 0, e->st, tiles, stride, (const double*)e->part, out);
+// losses of the held steps s0 .. s0 + steps
+static void launch_loss(mpcx_mlp* e, int tiles, long long s0, long long steps, double* out) {
+  hipLaunchKernelGGL(loss_sums, dim3((unsigned)steps), dim3(64), 0, e->st, tiles, part_stride(e),
+                     (const double*)(e->part + s0 * part_stride(e)), out);
 }
 static int loss_tiles(const mpcx_mlp* e, int rows) { return (up32(rows) / 16) * ((e->n_out + 15) / 16); }
 
@@ -631,12 +640,13 @@ extern "C" int mpcx_mlp_loss_grad(mpcx_mlp* e, int32_t rows, const float* x, con
                                   double* loss, float* grad) {
   if (!e || rows < 1 || !x || !target || !wout || !loss) return set_error(MPCX_E_ARG, "bad arguments");
   int rc;
-  if ((rc = train_buffers(e, rows, 1)) || (rc = upload_data(e, rows, x, target, wout)) ||
+  long long held;
+  if ((rc = train_buffers(e, rows, 1, held)) || (rc = upload_data(e, rows, x, target, wout)) ||
       (rc = grow(e->st, e->loss, e->loss_n, 1)))
     return rc;
   launch_inputs(e, rows, rows, 1, nullptr);
   train_step(e, rows, 0, e->T, nullptr, e->W, Adam{});
-  launch_loss(e, loss_tiles(e, rows), 1, e->loss);
+  launch_loss(e, loss_tiles(e, rows), 0, 1, e->loss);
   MLCHK(hipMemcpyAsync(loss, e->loss, 8, hipMemcpyDeviceToHost, e->st));
   if (grad) MLCHK(hipMemcpyAsync(grad, e->g, e->nparam * 4, hipMemcpyDeviceToHost, e->st));
   MLCHK(hipStreamSynchronize(e->st));
@@ -656,7 +666,8 @@ extern "C" int mpcx_mlp_train(mpcx_mlp* e, int64_t n, const float* x, const floa
   const long long steps = (n + batch - 1) / batch;
   const int CHUNK = (int)std::max<int64_t>(1, std::min<int64_t>(64, (1 << 22) / n));   // epochs whose orders are uploaded together
   int rc;
-  if ((rc = train_buffers(e, batch, steps)) || (rc = upload_data(e, n, x, target, wout)) ||
+  long long held;
+  if ((rc = train_buffers(e, batch, steps, held)) || (rc = upload_data(e, n, x, target, wout)) ||
       (rc = grow(e->st, e->idx, e->idx_n, n * CHUNK)) || (rc = grow(e->st, e->loss, e->loss_n, steps * std::max(epochs, 1))))
     return rc;
   std::vector<int> order((size_t)n * std::min(CHUNK, std::max(epochs, 1)));
@@ -684,17 +695,18 @@ extern "C" int mpcx_mlp_train(mpcx_mlp* e, int64_t n, const float* x, const floa
     for (int q = 0; q < ne && !rc; q++) {
       const int* idx = e->idx + (size_t)q * n;
       double* lo = e->loss + (size_t)(e0 + q) * steps;
-      launch_inputs(e, n, batch, steps, idx);
-      for (long long s = 0; s < steps; s++) {
-        e->t += 1;
-        const float c1 = 1.f - powf(0.9f, (float)e->t), c2 = 1.f - powf(0.999f, (float)e->t);
-        train_step(e, s + 1 < steps ? batch : tail, s, e->T, idx + s * batch, e->W,
-                   Adam{lr, 0.9f, 0.999f, 1e-8f, c1, c2, 1});
+      for (long long s0 = 0; s0 < steps; s0 += held) {
+        const long long ns = std::min(held, steps - s0), full = s0 + ns < steps ? ns : ns - 1;
+        launch_inputs(e, n - s0 * batch, batch, ns, idx + s0 * batch);
+        for (long long s = 0; s < ns; s++) {
+          e->t += 1;
+          const float c1 = 1.f - powf(0.9f, (float)e->t), c2 = 1.f - powf(0.999f, (float)e->t);
+          train_step(e, s < full ? batch : tail, s, e->T, idx + (s0 + s) * batch, e->W,
+                     Adam{lr, 0.9f, 0.999f, 1e-8f, c1, c2, 1});
+        }
+        if (full) launch_loss(e, loss_tiles(e, batch), 0, full, lo + s0);
+        if (full < ns) launch_loss(e, loss_tiles(e, tail), full, 1, lo + s0 + full);
       }
-      if (steps > 1) launch_loss(e, loss_tiles(e, batch), steps - 1, lo);
-      hipLaunchKernelGGL(loss_sums, dim3(1), dim3(64), 0, e->st, loss_tiles(e, tail), 0ll,
-                         (const double*)(e->part + (steps - 1) * ((long long)(up32(e->cap) / 16) * ((e->n_out + 15) / 16) + 4)),
-                         lo + steps - 1);
     }
   }
   (void)hipEventRecord(a1, e->st);
