@@ -3245,7 +3245,7 @@ struct mpcx_co {
 template <typename T>
 static T* dalloc(mpcx_co* e, size_t n) {
   void* p = nullptr;
-  if (hipMalloc(&p, n * sizeof(T) + 64) != hipSuccess) return nullptr;
+  if (mpcx::device_alloc(&p, n * sizeof(T) + 64) != hipSuccess) return nullptr;
   e->allocs.push_back(p);
   return (T*)p;
 }
@@ -4258,7 +4258,7 @@ extern "C" int mpcx_co_init_solvent(mpcx_co* e, int64_t Na0, int64_t Nb0, double
   if (!e || Na0 < 0 || Nb0 < 0 || Na0 + Nb0 > e->P.NT || !(T >= 0)) return set_error(MPCX_E_ARG, "bad arguments");
   const int nblk = 2048;
   double* part = nullptr;
-  HIPCHK(hipMalloc(&part, (size_t)nblk * 3 * 8));
+  HIPCHK(mpcx::device_alloc(&part, (size_t)nblk * 3 * 8));
   hipLaunchKernelGGL(init_solvent, dim3(nblk), dim3(256), 0, e->st, e->P, e->D, (long long)Na0, (long long)Nb0,
                      sqrt(T / e->cfg.Ma), sqrt(T / e->cfg.Mb), sqrt(T / e->cfg.Ms), (unsigned long long)seed, part);
   hipLaunchKernelGGL(init_zero_momentum, dim3(1024), dim3(256), 0, e->st, e->P, e->D, (const double*)part, nblk);
@@ -5764,16 +5764,16 @@ static int cob_tiles(mpcx_cob* b) {
   }
   for (Tile** d : {&b->d_pt, &b->d_ct, &b->d_vt, &b->d_gt, &b->d_xt, &b->d_nt})
     if (*d) { (void)hipFree(*d); *d = nullptr; }
-  HIPCHK(hipMalloc(&b->d_xt, xt.size() * sizeof(Tile)));
-  HIPCHK(hipMalloc(&b->d_nt, nt.size() * sizeof(Tile)));
+  HIPCHK(mpcx::device_alloc(&b->d_xt, xt.size() * sizeof(Tile)));
+  HIPCHK(mpcx::device_alloc(&b->d_nt, nt.size() * sizeof(Tile)));
   HIPCHK(hipMemcpy(b->d_xt, xt.data(), xt.size() * sizeof(Tile), hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(b->d_nt, nt.data(), nt.size() * sizeof(Tile), hipMemcpyHostToDevice));
   b->n_xt = (int)xt.size();
   b->n_nt = (int)nt.size();
-  HIPCHK(hipMalloc(&b->d_pt, pt.size() * sizeof(Tile)));
-  HIPCHK(hipMalloc(&b->d_gt, gt.size() * sizeof(Tile)));
-  HIPCHK(hipMalloc(&b->d_ct, ct.size() * sizeof(Tile)));
-  HIPCHK(hipMalloc(&b->d_vt, vt.size() * sizeof(Tile)));
+  HIPCHK(mpcx::device_alloc(&b->d_pt, pt.size() * sizeof(Tile)));
+  HIPCHK(mpcx::device_alloc(&b->d_gt, gt.size() * sizeof(Tile)));
+  HIPCHK(mpcx::device_alloc(&b->d_ct, ct.size() * sizeof(Tile)));
+  HIPCHK(mpcx::device_alloc(&b->d_vt, vt.size() * sizeof(Tile)));
   HIPCHK(hipMemcpy(b->d_gt, gt.data(), gt.size() * sizeof(Tile), hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(b->d_pt, pt.data(), pt.size() * sizeof(Tile), hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(b->d_ct, ct.data(), ct.size() * sizeof(Tile), hipMemcpyHostToDevice));
@@ -5793,10 +5793,10 @@ static int cob_tiles(mpcx_cob* b) {
     b->icap = b->icap_set > 0 ? b->icap_set : std::max(b->tile / 2, 256);
     if (n * (long long)b->icap > (1ll << 31)) return set_error(MPCX_E_ARG, "too many particle tiles for the inboxes");
     b->n_tiles = (int)n;
-    HIPCHK(hipMalloc(&b->d_tb, b->R * sizeof(int)));
-    HIPCHK(hipMalloc(&b->d_icnt, n * sizeof(int)));
-    HIPCHK(hipMalloc(&b->d_ibox, n * (size_t)b->icap * sizeof(FxEntry)));
-    HIPCHK(hipMalloc(&b->d_orng, n * sizeof(int2)));
+    HIPCHK(mpcx::device_alloc(&b->d_tb, b->R * sizeof(int)));
+    HIPCHK(mpcx::device_alloc(&b->d_icnt, n * sizeof(int)));
+    HIPCHK(mpcx::device_alloc(&b->d_ibox, n * (size_t)b->icap * sizeof(FxEntry)));
+    HIPCHK(mpcx::device_alloc(&b->d_orng, n * sizeof(int2)));
     HIPCHK(hipMemcpy(b->d_tb, tb.data(), b->R * sizeof(int), hipMemcpyHostToDevice));
     HIPCHK(hipMemset(b->d_icnt, 0, n * sizeof(int)));
   }
@@ -6103,9 +6103,9 @@ static int cob_make(mpcx_cob** out, int32_t R, mpcx_co* const* engines, int32_t 
              hipStreamCreateWithFlags(&b->st2, hipStreamNonBlocking) != hipSuccess) {
     rc = set_error(MPCX_E_HIP, "batch stream creation failed");
   }
-  if (!rc && (hipMalloc(&b->d_P, R * sizeof(CoP)) != hipSuccess || hipMalloc(&b->d_D, R * sizeof(CoD)) != hipSuccess ||
-              hipMalloc(&b->d_X, R * sizeof(CoSortD)) != hipSuccess || hipMalloc(&b->d_S, R * sizeof(SpD)) != hipSuccess ||
-              hipMalloc(&b->d_N, R * sizeof(SpD)) != hipSuccess || hipMalloc(&b->d_io, R * sizeof(int)) != hipSuccess ||
+  if (!rc && (mpcx::device_alloc(&b->d_P, R * sizeof(CoP)) != hipSuccess || mpcx::device_alloc(&b->d_D, R * sizeof(CoD)) != hipSuccess ||
+              mpcx::device_alloc(&b->d_X, R * sizeof(CoSortD)) != hipSuccess || mpcx::device_alloc(&b->d_S, R * sizeof(SpD)) != hipSuccess ||
+              mpcx::device_alloc(&b->d_N, R * sizeof(SpD)) != hipSuccess || mpcx::device_alloc(&b->d_io, R * sizeof(int)) != hipSuccess ||
               hipEventCreate(&b->e0) != hipSuccess ||
               hipEventCreate(&b->e1) != hipSuccess ||
               hipEventCreateWithFlags(&b->fork, hipEventDisableTiming) != hipSuccess ||
@@ -6417,7 +6417,7 @@ extern "C" int mpcx_cob_body_average(mpcx_cob* b, int64_t n, int32_t nr, int32_t
   unsigned* acc = nullptr;
   double* vacc = nullptr;
   int rc = 0;
-  if (hipMalloc(&acc, bins * 4) != hipSuccess || hipMalloc(&vacc, b->R * 8) != hipSuccess ||
+  if (mpcx::device_alloc(&acc, bins * 4) != hipSuccess || mpcx::device_alloc(&vacc, b->R * 8) != hipSuccess ||
       hipMemcpy(acc, counts, bins * 4, hipMemcpyHostToDevice) != hipSuccess ||
       hipMemcpy(vacc, vsum, b->R * 8, hipMemcpyHostToDevice) != hipSuccess)
     rc = set_error(MPCX_E_HIP, "body accumulator allocation failed");

@@ -90,7 +90,7 @@ extern "C" int mpcx_philox_uniform2(uint64_t seed, uint32_t stream, uint64_t ste
     return mpcx::set_error(MPCX_E_ARG, "bad arguments (n <= 2^28, stream < 65536)");
   if (n == 0) return 0;
   double* d = nullptr;
-  if (hipMalloc(&d, (size_t)n * 16) != hipSuccess) return mpcx::set_error(MPCX_E_HIP, "hipMalloc failed");
+  if (mpcx::device_alloc(&d, (size_t)n * 16) != hipSuccess) return mpcx::set_error(MPCX_E_HIP, "hipMalloc failed");
   hipLaunchKernelGGL(philox_fill_kernel, dim3(1024), dim3(256), 0, 0, seed, stream, step, idx0, (long long)n, d);
   hipError_t r = hipGetLastError();
   if (r == hipSuccess) r = hipMemcpy(out, d, (size_t)n * 16, hipMemcpyDeviceToHost);
@@ -104,7 +104,7 @@ extern "C" int mpcx_probe_copy(int64_t nbytes, int32_t reps, double* ms_per_copy
   void *a = nullptr, *b = nullptr;
   hipEvent_t e0 = nullptr, e1 = nullptr;
   int rc = 0;
-  if (hipMalloc(&a, n * 16) != hipSuccess || hipMalloc(&b, n * 16) != hipSuccess) {
+  if (mpcx::device_alloc(&a, n * 16) != hipSuccess || mpcx::device_alloc(&b, n * 16) != hipSuccess) {
     rc = mpcx::set_error(MPCX_E_HIP, "hipMalloc failed");
   } else {
     (void)hipMemset(a, 0, n * 16);

@@ -15,6 +15,7 @@
 #include <vector>
 #include "mpcx_device.h"
 #include "mpcx_host.h"
+#include "mpcx_stage.h"
 #include "../../include/mpcx.h"
 
 #pragma clang fp contract(off)
@@ -180,7 +181,7 @@ static int observables(const DevView& v, double* out, bool selkov) {
   hipStream_t st = (hipStream_t)v.stream;
   const int g = grid_n(v.n);
   double* part = nullptr;
-  DGCHK(hipMalloc(&part, (size_t)g * 7 * 8));
+  DGCHK(mpcx::device_alloc(&part, (size_t)g * 7 * 8));
   hipLaunchKernelGGL(dg_sums, dim3(g), dim3(DT), 0, st, kview(v), part);
   std::vector<double> h((size_t)g * 7);
   hipError_t r = hipMemcpyAsync(h.data(), part, h.size() * 8, hipMemcpyDeviceToHost, st);
@@ -255,7 +256,7 @@ static int body_density(const DevView& v, int dimer, int nr, int nz, double rmax
   B.rmax = rmax; B.zmin = zmin; B.zmax = zmax; B.nr = nr; B.nz = nz; B.periodic_z = v.periodic_z;
   const size_t bins = (size_t)3 * nz * nr;
   unsigned* h = nullptr;
-  DGCHK(hipMalloc(&h, bins * 4));
+  DGCHK(mpcx::device_alloc(&h, bins * 4));
   hipError_t r = hipMemsetAsync(h, 0, bins * 4, st);
   if (r == hipSuccess) {
     hipLaunchKernelGGL(dg_body, dim3(grid_n(v.n)), dim3(DT), 0, st, kview(v), B, h);
@@ -299,7 +300,7 @@ extern "C" int mpcx_co_conc_slabs(mpcx_co* e, double x_slab, double y_slab, doub
   const size_t n = 2 * ((size_t)S.nx + (size_t)S.nx * S.ny + (size_t)S.nx * S.nz + (size_t)S.ny * S.nz);
   hipStream_t st = (hipStream_t)v.stream;
   int* d = nullptr;
-  DGCHK(hipMalloc(&d, n * 4));
+  DGCHK(mpcx::device_alloc(&d, n * 4));
   hipError_t r = hipMemsetAsync(d, 0, n * 4, st);
   if (r == hipSuccess) {
     hipLaunchKernelGGL(dg_slabs, dim3(grid_n(v.n)), dim3(DT), 0, st, kview(v), S, d);
@@ -318,7 +319,7 @@ extern "C" int mpcx_sk_shells(mpcx_sk* e, int64_t* counts24) {
   if (rc) return rc;
   hipStream_t st = (hipStream_t)v.stream;
   long long* d = nullptr;
-  DGCHK(hipMalloc(&d, 24 * 8));
+  DGCHK(mpcx::device_alloc(&d, 24 * 8));
   hipError_t r = hipMemsetAsync(d, 0, 24 * 8, st);
   if (r == hipSuccess) {
     hipLaunchKernelGGL(dg_shells, dim3(grid_n(v.n)), dim3(DT), 0, st, kview(v), v.dim[0][0], v.dim[1][0], v.dim[2][0], d);

@@ -381,7 +381,7 @@ static int grow(hipStream_t st, T*& q, long long& have, long long n) {
   if (n <= have) return 0;
   release(q);
   have = 0;
-  MLCHK(hipMalloc(&q, (size_t)n * sizeof(T)));
+  MLCHK(mpcx::device_alloc(&q, (size_t)n * sizeof(T)));
   MLCHK(hipMemsetAsync(q, 0, (size_t)n * sizeof(T), st));
   have = n;
   return 0;
@@ -533,8 +533,8 @@ extern "C" int mpcx_mlp_create(mpcx_mlp** out, int32_t n_in, int32_t n_hidden, i
     }
   }
   if (hipStreamCreateWithFlags(&e->st, hipStreamNonBlocking) != hipSuccess ||
-      hipMalloc(&e->p, o * 4) != hipSuccess || hipMalloc(&e->g, o * 4) != hipSuccess ||
-      hipMalloc(&e->m, o * 4) != hipSuccess || hipMalloc(&e->v, o * 4) != hipSuccess) {
+      mpcx::device_alloc(&e->p, o * 4) != hipSuccess || mpcx::device_alloc(&e->g, o * 4) != hipSuccess ||
+      mpcx::device_alloc(&e->m, o * 4) != hipSuccess || mpcx::device_alloc(&e->v, o * 4) != hipSuccess) {
     mpcx_mlp_destroy(e);
     return set_error(MPCX_E_HIP, "device allocation failed");
   }
@@ -589,8 +589,8 @@ extern "C" int mpcx_mlp_forward(mpcx_mlp* e, int32_t rows, const float* x, float
     e->Fb.assign(L - 1, nullptr);
     for (int l = 0; l + 1 < L; l++)
       if ((rc = zeroed(e->st, e->Fb[l], (size_t)Rp * up32(e->dims[l])))) return rc;
-    MLCHK(hipMalloc(&e->Fx, (size_t)rows * e->n_in * 4));
-    MLCHK(hipMalloc(&e->Fy, (size_t)rows * e->n_out * 4));
+    MLCHK(mpcx::device_alloc(&e->Fx, (size_t)rows * e->n_in * 4));
+    MLCHK(mpcx::device_alloc(&e->Fy, (size_t)rows * e->n_out * 4));
     e->fcap = rows;
   }
   MLCHK(hipMemcpyAsync(e->Fx, x, (size_t)rows * e->n_in * 4, hipMemcpyHostToDevice, e->st));
@@ -750,9 +750,9 @@ extern "C" int mpcx_gemm_bf16(int32_t M, int32_t N, int32_t K, const float* A, c
   const int Mp = up32(M), Np = up32(N), Kp = up32(K);
   float *Af = nullptr, *Bf = nullptr, *Cd = nullptr;
   __bf16 *Ab = nullptr, *Bb = nullptr;
-  MLCHK(hipMalloc(&Af, (size_t)M * K * 4)); MLCHK(hipMalloc(&Bf, (size_t)K * N * 4));
-  MLCHK(hipMalloc(&Ab, (size_t)Mp * Kp * 2)); MLCHK(hipMalloc(&Bb, (size_t)Np * Kp * 2));
-  MLCHK(hipMalloc(&Cd, (size_t)M * N * 4));
+  MLCHK(mpcx::device_alloc(&Af, (size_t)M * K * 4)); MLCHK(mpcx::device_alloc(&Bf, (size_t)K * N * 4));
+  MLCHK(mpcx::device_alloc(&Ab, (size_t)Mp * Kp * 2)); MLCHK(mpcx::device_alloc(&Bb, (size_t)Np * Kp * 2));
+  MLCHK(mpcx::device_alloc(&Cd, (size_t)M * N * 4));
   MLCHK(hipMemset(Ab, 0, (size_t)Mp * Kp * 2));
   MLCHK(hipMemset(Bb, 0, (size_t)Np * Kp * 2));
   MLCHK(hipMemcpy(Af, A, (size_t)M * K * 4, hipMemcpyHostToDevice));

@@ -1455,7 +1455,7 @@ struct mpcx_sk {
 template <typename T>
 static T* skalloc(mpcx_sk* e, size_t n) {
   void* p = nullptr;
-  if (hipMalloc(&p, n * sizeof(T) + 64) != hipSuccess) return nullptr;
+  if (mpcx::device_alloc(&p, n * sizeof(T) + 64) != hipSuccess) return nullptr;
   e->allocs.push_back(p);
   return (T*)p;
 }
@@ -1690,7 +1690,7 @@ extern "C" int mpcx_sk_run(mpcx_sk* e, int64_t ncoll, const double* draws, int64
     if (!draws || ndraws < 1) return set_error(MPCX_E_ARG, "rng_mode 0 needs host draws");
     if (ndraws > e->nU_cap) {
       void* p = nullptr;
-      if (hipMalloc(&p, ndraws * 8) != hipSuccess) return set_error(MPCX_E_HIP, "hipMalloc failed");
+      if (mpcx::device_alloc(&p, ndraws * 8) != hipSuccess) return set_error(MPCX_E_HIP, "hipMalloc failed");
       e->allocs.push_back(p);
       e->d_U = (double*)p;
       e->nU_cap = ndraws;

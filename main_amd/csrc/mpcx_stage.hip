@@ -251,20 +251,38 @@ struct Block {
   int dev;
 };
 std::mutex g_blocks_mu;
-std::vector<Block> g_blocks;   // free blocks, at most CACHE_MAX bytes
+std::deque<Block> g_blocks;   // free blocks, the longest unused first, at most CACHE_MAX bytes
 size_t g_blocks_bytes = 0;
 constexpr size_t CACHE_MAX = 512u << 20;
+
+size_t block_bytes(size_t n) { return (std::max<size_t>(n, 256) + 255) / 256 * 256; }
 
 }  // namespace
 
 int copy_out(const std::vector<HostCopy>& v, hipStream_t st) { return copy(v, true, st); }
 int copy_in(const std::vector<HostCopy>& v, hipStream_t st) { return copy(v, false, st); }
 
+// Every device allocation of the library comes through here: memory that only
+// the cache holds must not make one fail.
+hipError_t device_alloc_bytes(void** p, size_t n) {
+  hipError_t r = hipMalloc(p, n);
+  if (r == hipSuccess) return r;
+  (void)hipGetLastError();
+  {
+    std::lock_guard<std::mutex> l(g_blocks_mu);
+    if (g_blocks.empty()) return r;
+  }
+  blocks_release();
+  r = hipMalloc(p, n);
+  if (r != hipSuccess) (void)hipGetLastError();
+  return r;
+}
+
 // The smallest free block that holds n bytes and is at most twice that (a new
 // one otherwise).  The entry points that use these run on the null stream, so
 // a block's next user is ordered after its last.
 void* block_get(size_t n, size_t* got) {
-  n = (std::max<size_t>(n, 256) + 255) / 256 * 256;
+  n = block_bytes(n);
   int dev = -1;
   if (hipGetDevice(&dev) != hipSuccess) return nullptr;
   {
@@ -283,26 +301,30 @@ void* block_get(size_t n, size_t* got) {
     }
   }
   void* p = nullptr;
-  if (hipMalloc(&p, n) != hipSuccess) {
-    (void)hipGetLastError();
-    blocks_release();   // make room, once
-    if (hipMalloc(&p, n) != hipSuccess) return nullptr;
-  }
+  if (device_alloc_bytes(&p, n) != hipSuccess) return nullptr;
   *got = n;
   return p;
 }
+// A block that does not fit drives out the longest unused ones: a driver that
+// goes on with another system's sizes keeps those, not the last system's.
 void block_put(void* p, size_t n) {
   if (!p) return;
   int dev = -1;
-  if (hipGetDevice(&dev) == hipSuccess) {
+  std::vector<void*> out;
+  const bool keep = n <= CACHE_MAX && hipGetDevice(&dev) == hipSuccess;
+  if (keep) {
     std::lock_guard<std::mutex> l(g_blocks_mu);
-    if (g_blocks_bytes + n <= CACHE_MAX) {
-      g_blocks.push_back(Block{p, n, dev});
-      g_blocks_bytes += n;
-      return;
+    while (g_blocks_bytes + n > CACHE_MAX) {
+      out.push_back(g_blocks.front().p);
+      g_blocks_bytes -= g_blocks.front().n;
+      g_blocks.pop_front();
     }
+    g_blocks.push_back(Block{p, n, dev});
+    g_blocks_bytes += n;
+  } else {
+    out.push_back(p);
   }
-  (void)hipFree(p);
+  for (void* q : out) (void)hipFree(q);
 }
 void blocks_release() {
   std::lock_guard<std::mutex> l(g_blocks_mu);

@@ -1,0 +1,64 @@
+"""The device blocks the drop-ins keep between calls (main_amd/csrc/mpcx_stage.hip),
+on the host with a device heap of a set size: bounded, the longest unused go
+first, and given back when anything else of the library finds no memory."""
+import ctypes as C
+import glob
+import os
+import re
+
+import pytest
+
+from tests.stage_host import HERE, Stage
+
+MB = 1 << 20
+
+
+@pytest.fixture(scope="module")
+def stage(tmp_path_factory):
+    return Stage(tmp_path_factory.mktemp("stage"))
+
+
+def test_blocks_are_reused(stage):
+    stage.reset()
+    a = stage.get(10 * MB)
+    stage.put(a)
+    assert stage.get(9 * MB) == a and stage.c.t_mallocs() == 1
+
+
+def test_another_size_drives_out_the_longest_unused(stage):
+    """600 MB of one system's blocks, then calls of another size: kept from the first on."""
+    stage.reset()
+    old = [stage.get(100 * MB) for _ in range(6)]
+    for b in old:
+        stage.put(b)
+    assert stage.c.t_used() <= 512 * MB
+    for _ in range(2):
+        new = [stage.get(30 * MB) for _ in range(3)]
+        for b in new:
+            stage.put(b)
+        assert stage.c.t_used() <= 512 * MB
+    assert stage.c.t_mallocs() == 9   # the second call's come from the first's
+    assert stage.get(100 * MB) in old[2:]   # and the newer ones of the old are still there
+    stage.reset()
+    big = stage.get(600 * MB)
+    stage.put(big)   # more than the cache holds: straight back
+    assert stage.c.t_used() == 0
+
+
+def test_an_allocation_takes_the_cached_memory_back(stage):
+    stage.reset(heap=1000 * MB)
+    for b in [stage.get(100 * MB) for _ in range(5)]:
+        stage.put(b)
+    p = stage.c.t_alloc(800 * MB)
+    assert p is not None and stage.c.t_used() == 800 * MB
+    assert stage.c.t_alloc(300 * MB) is None   # nothing left to give back: an error, as hipMalloc's
+    stage.c.t_free(C.c_void_p(p))
+
+
+def test_every_allocation_goes_through_it():
+    for path in glob.glob(os.path.join(HERE, "..", "main_amd", "csrc", "*")):
+        if os.path.basename(path) == "mpcx_stage.hip":
+            continue
+        with open(path) as f:
+            code = re.sub(r"//[^\n]*|\"[^\"\n]*\"", "", f.read())
+        assert "hipMalloc(" not in code, path
