@@ -40,18 +40,23 @@ struct Ring {
 };
 Ring g_ring;
 
-void ring_release() {
-  if (g_ring.pin) (void)hipHostFree(g_ring.pin);
-  g_ring.pin = nullptr;
+void events_release() {
   for (auto& e : g_ring.ev) {
     if (e) (void)hipEventDestroy(e);
     e = nullptr;
   }
   g_ring.dev = -1;
 }
+void ring_release() {
+  if (g_ring.pin) (void)hipHostFree(g_ring.pin);
+  g_ring.pin = nullptr;
+  events_release();
+}
 // the ring on the current device, or false (the caller copies plainly): no
 // pinned memory to be had, or a stream of another device, whose work the
-// ring's events cannot mark
+// ring's events cannot mark.  The slots serve every device; only the events
+// are made anew for another one (pinning 32 MB takes as long as 100 MB of
+// copies).
 bool ring_ready(hipStream_t st) {
   int dev = -1, sdev = -1;
   if (hipGetDevice(&dev) != hipSuccess) return false;
@@ -59,18 +64,18 @@ bool ring_ready(hipStream_t st) {
     (void)hipGetLastError();
     return false;
   }
-  if (g_ring.pin && g_ring.dev == dev) return true;
-  ring_release();
-  if (hipHostMalloc((void**)&g_ring.pin, SLOT * NSLOT, hipHostMallocDefault) != hipSuccess) {
+  if (!g_ring.pin && hipHostMalloc((void**)&g_ring.pin, SLOT * NSLOT, hipHostMallocPortable) != hipSuccess) {
     g_ring.pin = nullptr;
     (void)hipGetLastError();
     return false;
   }
+  if (g_ring.dev == dev) return true;
+  events_release();
   for (auto& e : g_ring.ev)
     if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
       e = nullptr;
       (void)hipGetLastError();
-      ring_release();
+      events_release();
       return false;
     }
   g_ring.dev = dev;

@@ -90,3 +90,15 @@ def test_pinned_arrays_go_straight_over_the_link(stage, out):
         assert np.array_equal(dst[k], src[k])
     if out:
         assert np.array_equal(wide, dev[2])
+
+
+def test_the_ring_serves_one_device_after_another(stage):
+    stage.reset()
+    a, b = rng_bytes(40 * MB + 8, 1), np.zeros(40 * MB + 8, np.uint8)
+    for k in range(4):
+        stage.c.t_device(k % 2)
+        b[:] = 0
+        assert stage.copy([b], [a], 1) == 0 and np.array_equal(a, b)
+    assert stage.c.t_host_mallocs() == 1 and stage.c.t_events() == 16
+    stage.reset()
+    assert stage.c.t_events() == 0
