@@ -15,8 +15,9 @@
 #include <atomic>
 #include <condition_variable>
 #include <deque>
+#include <exception>
 #include <mutex>
-#include <system_error>
+#include <new>
 #include <thread>
 #include <vector>
 #include "mpcx_host.h"
@@ -55,8 +56,7 @@ void ring_release() {
 // the ring on the current device, or false (the caller copies plainly): no
 // pinned memory to be had, or a stream of another device, whose work the
 // ring's events cannot mark.  The slots serve every device; only the events
-// are made anew for another one (pinning 32 MB takes as long as 100 MB of
-// copies).
+// are made anew for another one.
 bool ring_ready(hipStream_t st) {
   int dev = -1, sdev = -1;
   if (hipGetDevice(&dev) != hipSuccess) return false;
@@ -99,15 +99,16 @@ void move_out(const Chunk& c, const char* slot) {
 }
 
 // Host threads that move slots; with none (small copies, or no thread to be
-// had) the caller's thread does it in post().
+// had) the caller's thread does it in post().  Nothing here allocates once the
+// threads run: a slot has at most one job.
 class Movers {
  public:
   explicit Movers(int n) {
     for (auto& b : busy_) b.store(0);
-    for (int i = 0; i < n; i++) {
+    for (; n_ < n; n_++) {
       try {
-        th_.emplace_back([this] { work(); });
-      } catch (const std::system_error&) {
+        th_[n_] = std::thread([this] { work(); });
+      } catch (const std::exception&) {   // no thread or no memory for it
         break;
       }
     }
@@ -118,17 +119,17 @@ class Movers {
       stop_ = true;
     }
     cv_.notify_all();
-    for (auto& t : th_) t.join();
+    for (int i = 0; i < n_; i++) th_[i].join();
   }
   void post(int slot, const Chunk& c, bool out) {
-    if (th_.empty()) {
+    if (n_ == 0) {
       run(slot, c, out);
       return;
     }
     busy_[slot].store(1);
     {
       std::lock_guard<std::mutex> l(mu_);
-      q_.push_back(Job{slot, c, out});
+      q_[tail_++ % NSLOT] = Job{slot, c, out};
     }
     cv_.notify_one();
   }
@@ -139,7 +140,11 @@ class Movers {
   }
 
  private:
-  struct Job { int slot; Chunk c; bool out; };
+  struct Job {
+    int slot;
+    Chunk c;
+    bool out;
+  };
   static void run(int slot, const Chunk& c, bool out) {
     char* p = g_ring.pin + (size_t)slot * SLOT;
     if (out) move_out(c, p);
@@ -148,10 +153,9 @@ class Movers {
   void work() {
     std::unique_lock<std::mutex> l(mu_);
     while (true) {
-      cv_.wait(l, [&] { return stop_ || !q_.empty(); });
-      if (q_.empty()) return;
-      const Job j = q_.front();
-      q_.pop_front();
+      cv_.wait(l, [&] { return stop_ || head_ != tail_; });
+      if (head_ == tail_) return;
+      const Job j = q_[head_++ % NSLOT];
       l.unlock();
       run(j.slot, j.c, j.out);
       l.lock();
@@ -159,8 +163,10 @@ class Movers {
       done_.notify_all();
     }
   }
-  std::vector<std::thread> th_;
-  std::deque<Job> q_;
+  std::thread th_[MAX_WORKERS];
+  int n_ = 0;
+  Job q_[NSLOT];
+  unsigned head_ = 0, tail_ = 0;
   std::mutex mu_;
   std::condition_variable cv_, done_;
   bool stop_ = false;
@@ -284,8 +290,17 @@ size_t block_bytes(size_t n) { return (std::max<size_t>(n, 256) + 255) / 256 * 2
 
 }  // namespace
 
-int copy_out(const std::vector<HostCopy>& v, hipStream_t st) { return copy(v, true, st); }
-int copy_in(const std::vector<HostCopy>& v, hipStream_t st) { return copy(v, false, st); }
+// (called below C entry points: no exception may pass)
+static int copy_noexcept(const std::vector<HostCopy>& v, bool out, hipStream_t st) {
+  try {
+    return copy(v, out, st);
+  } catch (const std::bad_alloc&) {
+    (void)hipStreamSynchronize(st);   // copies on their way still use the caller's arrays
+    return set_error(MPCX_E_HIP, "out of host memory");
+  }
+}
+int copy_out(const std::vector<HostCopy>& v, hipStream_t st) { return copy_noexcept(v, true, st); }
+int copy_in(const std::vector<HostCopy>& v, hipStream_t st) { return copy_noexcept(v, false, st); }
 
 // Every device allocation of the library comes through here: memory that only
 // the cache holds must not make one fail.
@@ -335,21 +350,22 @@ void* block_get(size_t n, size_t* got) {
 void block_put(void* p, size_t n) {
   if (!p) return;
   int dev = -1;
-  std::vector<void*> out;
-  const bool keep = n <= CACHE_MAX && hipGetDevice(&dev) == hipSuccess;
-  if (keep) {
+  bool kept = false;
+  if (n <= CACHE_MAX && hipGetDevice(&dev) == hipSuccess) {
     std::lock_guard<std::mutex> l(g_blocks_mu);
     while (g_blocks_bytes + n > CACHE_MAX) {
-      out.push_back(g_blocks.front().p);
+      (void)hipFree(g_blocks.front().p);
       g_blocks_bytes -= g_blocks.front().n;
       g_blocks.pop_front();
     }
-    g_blocks.push_back(Block{p, n, dev});
-    g_blocks_bytes += n;
-  } else {
-    out.push_back(p);
+    try {
+      g_blocks.push_back(Block{p, n, dev});
+      g_blocks_bytes += n;
+      kept = true;
+    } catch (const std::bad_alloc&) {   // (called by destructors)
+    }
   }
-  for (void* q : out) (void)hipFree(q);
+  if (!kept) (void)hipFree(p);
 }
 void blocks_release() {
   std::lock_guard<std::mutex> l(g_blocks_mu);

@@ -2,10 +2,23 @@
 // hip/hip_runtime.h beside this file; driven by tests/test_stage_host.py.
 #include <stdio.h>
 #include <stdlib.h>
-#include <deque>
 #include <map>
 #include <mutex>
+#include <atomic>
+#include <new>
 #include "../../main_amd/csrc/mpcx_stage.hip"
+
+static std::atomic<long> g_fail_at{-1};   // the allocation that fails (counted down; below 0: none)
+static bool fails() {
+  return g_fail_at.load() >= 0 && g_fail_at.fetch_sub(1) == 0;
+}
+void* operator new(size_t n) {
+  void* p = fails() ? nullptr : malloc(n ? n : 1);
+  if (!p) throw std::bad_alloc();
+  return p;
+}
+void operator delete(void* p) noexcept { free(p); }
+void operator delete(void* p, size_t) noexcept { free(p); }
 
 struct Copy {
   void* dst;
@@ -14,7 +27,7 @@ struct Copy {
 };
 struct StubStream {
   int dev = 0;
-  std::deque<Copy> q;    // copies not yet done
+  Copy q[4096];   // copies done .. queued are not yet made
   size_t done = 0, queued = 0;
 };
 struct StubEvent {
@@ -36,10 +49,9 @@ static bool within(const std::map<char*, size_t>& m, const void* p) {
   return it != m.begin() && (char*)p < std::prev(it)->first + std::prev(it)->second;
 }
 static void run_to(StubStream* s, size_t at) {
-  while (s->done < at) {
-    memcpy(s->q.front().dst, s->q.front().src, s->q.front().n);
-    s->q.pop_front();
-    s->done++;
+  for (; s->done < at; s->done++) {
+    const Copy& c = s->q[s->done % 4096];
+    memcpy(c.dst, c.src, c.n);
   }
 }
 #define LOCK std::lock_guard<std::recursive_mutex> lock(g_mu)
@@ -75,12 +87,12 @@ hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
 hipError_t hipHostFree(void* p) { free(p); return hipSuccess; }
 hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
   LOCK;
-  *e = new StubEvent();
+  *e = new (malloc(sizeof(StubEvent))) StubEvent();   // (the stand-in's own memory does not fail)
   (*e)->dev = g_dev;
   g_events++;
   return hipSuccess;
 }
-hipError_t hipEventDestroy(hipEvent_t e) { LOCK; delete e; g_events--; return hipSuccess; }
+hipError_t hipEventDestroy(hipEvent_t e) { LOCK; free(e); g_events--; return hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t e, hipStream_t st) {
   LOCK;
   if (e->dev != stream(st)->dev) return hipErrorInvalidValue;
@@ -92,8 +104,8 @@ hipError_t hipEventSynchronize(hipEvent_t e) { LOCK; if (e->st) run_to(e->st, e-
 hipError_t hipMemcpyAsync(void* dst, const void* src, size_t n, hipMemcpyKind kind, hipStream_t st) {
   LOCK;
   if (within(g_pinned, kind == hipMemcpyDeviceToHost ? dst : src)) g_direct += n;
-  stream(st)->q.push_back(Copy{dst, src, n});
-  stream(st)->queued++;
+  if (stream(st)->queued - stream(st)->done >= 4096) return hipErrorUnknown;
+  stream(st)->q[stream(st)->queued++ % 4096] = Copy{dst, src, n};
   return hipSuccess;
 }
 hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* p) {
@@ -133,10 +145,15 @@ void* t_alloc(size_t n) {
   return mpcx::device_alloc(&p, n) == hipSuccess ? p : nullptr;
 }
 void t_free(void* p) { (void)hipFree(p); }
-// n arrays between the host and "device" memory (here host memory too)
-int t_copy(int n, void** host, void** dev, const size_t* bytes, const int* widen, int out) {
+// n arrays between the host and "device" memory (here host memory too); the
+// result plus 1000 if the allocation to fail came up
+int t_copy(int n, void** host, void** dev, const size_t* bytes, const int* widen, int out, long fail_at) {
   std::vector<mpcx::HostCopy> v;
   for (int i = 0; i < n; i++) v.push_back(mpcx::HostCopy{host[i], dev[i], bytes[i], widen[i] != 0});
-  return out ? mpcx::copy_out(v, nullptr) : mpcx::copy_in(v, nullptr);
+  g_fail_at = fail_at;
+  const int rc = out ? mpcx::copy_out(v, nullptr) : mpcx::copy_in(v, nullptr);
+  const bool failed = fail_at >= 0 && g_fail_at < 0;
+  g_fail_at = -1;
+  return failed ? 1000 + rc : rc;
 }
 }

@@ -40,13 +40,14 @@ class Stage:
     def pin(self, a):
         self.c.t_pin(C.c_void_p(a.ctypes.data), C.c_size_t(a.nbytes))
 
-    def copy(self, host, dev, out, widen=None):
+    def copy(self, host, dev, out, widen=None, fail_at=-1):
         n = len(host)
         arr = lambda v, t: (t * n)(*v)
         widen = widen or [0] * n
         addr = lambda a: None if a is None else a.ctypes.data
         return self.c.t_copy(C.c_int(n), arr([addr(a) for a in host], C.c_void_p), arr([addr(a) for a in dev], C.c_void_p),
-                             arr([a.nbytes for a in dev], C.c_size_t), arr(widen, C.c_int), C.c_int(out))
+                             arr([a.nbytes for a in dev], C.c_size_t), arr(widen, C.c_int), C.c_int(out),
+                             C.c_long(fail_at))
 
 
 def rng_bytes(n, seed):

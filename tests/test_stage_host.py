@@ -102,3 +102,25 @@ def test_the_ring_serves_one_device_after_another(stage):
     assert stage.c.t_host_mallocs() == 1 and stage.c.t_events() == 16
     stage.reset()
     assert stage.c.t_events() == 0
+
+
+@pytest.mark.parametrize("out", [0, 1])
+@pytest.mark.parametrize("n", [4096, 9 * MB, 40 * MB])
+def test_no_exception_leaves_a_copy(stage, n, out):
+    """Each host allocation of a copy fails in turn: the copy is done without it
+    or returns an error, and the next one works."""
+    a, b = rng_bytes(n, 1), np.zeros(n, np.uint8)
+    w = np.zeros(MB, np.int64)
+    host = [b, w] if out else [a, None]
+    dev = [a if out else b, np.arange(MB, dtype=np.int32)]
+    for k in range(64):
+        stage.reset()
+        b[:] = 0
+        rc = stage.copy(host, dev, out, widen=[0, out], fail_at=k)
+        if rc < 500:
+            assert rc == 0
+            break   # no more than k allocations
+        assert rc < 1000 or np.array_equal(a, b)
+        b[:] = 0
+        assert stage.copy(host, dev, out, widen=[0, out]) == 0 and np.array_equal(a, b)
+    assert k >= 1
