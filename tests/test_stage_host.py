@@ -124,3 +124,21 @@ def test_no_exception_leaves_a_copy(stage, n, out):
         b[:] = 0
         assert stage.copy(host, dev, out, widen=[0, out]) == 0 and np.array_equal(a, b)
     assert k >= 1
+
+
+SLOT, LIMIT = 2 * MB, MB
+
+
+@pytest.mark.parametrize("out", [0, 1])
+@pytest.mark.parametrize("sizes", [[8], [LIMIT - 8], [LIMIT], [SLOT, SLOT + 8], [4 * SLOT - 8, 24, 4 * SLOT + 16], [16 * SLOT],
+                                   [16 * SLOT + 8], [7 * MB, 7 * MB, 7 * MB, 7 * MB, 7 * MB, 7 * MB + 8],
+                                   [33 * SLOT + 40], [50 * SLOT]])
+def test_copies_round_trip(stage, sizes, out):
+    """One array and several, up to three times round the ring, into and out of the device."""
+    stage.reset()
+    src = [rng_bytes(n, n) for n in sizes]
+    dst = [np.zeros(n, np.uint8) for n in sizes]
+    host, dev = (dst, src) if out else (src, dst)
+    assert stage.copy(host, dev, out) == 0
+    assert all(np.array_equal(a, b) for a, b in zip(src, dst))
+    assert stage.c.t_host_mallocs() == (1 if sum(sizes) >= LIMIT else 0)
