@@ -1,6 +1,7 @@
 """The surrogate's products at the edges of their tiles: sizes that are not
 multiples of 16 or 32, one row, ragged batches, more layers than one gradient
-launch takes, buffers reused after a larger batch.
+launch takes, buffers reused after a larger batch; and sizes on both sides of
+the 4,096 tiles of 16 x 16 from which a product takes tiles of 32 x 32.
 
 Tolerance: the reference rounds the same operands to BF16 and sums in FP64; the
 FP32 sums differ by about 1e-7, which moves about 1e-4 of the BF16 roundings of
@@ -10,7 +11,7 @@ deepest network here; asserted at 2e-3.
 import numpy as np
 import pytest
 
-from main_amd.surrogate import Surrogate
+from main_amd.surrogate import Surrogate, gemm_bf16
 from tests import mlp_reference as M
 
 pytestmark = pytest.mark.gpu
@@ -75,3 +76,35 @@ def test_an_epoch_is_adam_on_its_batches(n, batch):
     finally:
         net.close()
         twin.close()
+
+
+def _tiles(m, n):
+    return (m + 31) // 32 * 2 * ((n + 15) // 16)
+
+
+@pytest.mark.parametrize("m,n,k,wide", [(1000, 1008, 33, False), (1024, 1024, 32, True), (1037, 1045, 70, True),
+                                        (2049, 513, 1, True), (4097, 241, 64, True), (33, 32700, 45, True)])
+def test_products_of_wide_tiles(m, n, k, wide):
+    """FP32 sums of exact products of BF16 values: their rounding, as the small products'."""
+    assert (_tiles(m, n) >= 4096) == wide
+    rng = np.random.default_rng(m + n + k)
+    A, B = rng.normal(size=(m, k)).astype(np.float32), rng.normal(size=(k, n)).astype(np.float32)
+    C, _ = gemm_bf16(A, B)
+    a, b = M.to_bf16(A), M.to_bf16(B)
+    assert np.max(np.abs(C - a @ b) / (np.abs(a) @ np.abs(b))) < 1e-6
+
+
+@pytest.mark.parametrize("hidden,rows", [(256, (8192, 545, 1025, 480, 3)), (200, (4129, 5057, 512)), (31, (545, 97))])
+def test_screening_of_many_rows(hidden, rows):
+    """Batches one after the other on one network: wide tiles in some layers (480
+    rows: none; 545: the output layer; 5,057 and more: the hidden ones of 200
+    or 256 units too), buffers kept from a larger batch, ragged edges."""
+    net = Surrogate(n_in=8, n_hidden=hidden, n_layers=2, n_out=2049, seed=8)
+    try:
+        flat = net.params().astype(np.float64)
+        for n in rows:
+            x = np.random.default_rng(n).normal(size=(n, 8)).astype(np.float32)
+            H, _ = M.forward(flat, net.dims(), x.astype(np.float64), bf16=True)
+            assert np.max(np.abs(net.forward_raw(x) - H[-1])) <= 2e-3 * np.max(np.abs(H[-1])), n
+    finally:
+        net.close()
