@@ -47,12 +47,15 @@ def build_collective(p, seed=3, flags_mix=False, mt_seed=4357787):
 
 
 def close(a, b, scale):
+    """Values out of tolerance and the largest relative error; a NaN on either side is out of tolerance."""
     a = np.asarray(a, np.float64).ravel()
     b = np.asarray(b, np.float64).ravel()
-    tol = REL_TOL * np.maximum(np.abs(b), scale)
-    bad = np.abs(a - b) > tol
-    err = float(np.max(np.abs(a - b) / np.maximum(np.abs(b), scale))) if a.size else 0.0
-    return int(bad.sum()), err
+    ref = np.maximum(np.abs(b), scale)
+    with np.errstate(invalid="ignore", divide="ignore"):
+        d = np.where(a == b, 0.0, np.abs(a - b))
+        bad = ~((d <= REL_TOL * ref) & np.isfinite(d) | (a == b))
+        err = np.where(a == b, 0.0, d / ref)
+    return int(bad.sum()), float(np.max(err)) if a.size else 0.0
 
 
 def collective_parity_case(ncoll=1, seed=3, p=None, flags_mix=False, sort_at_setup=True, tour=None,
