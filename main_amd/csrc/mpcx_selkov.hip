@@ -1725,16 +1725,19 @@ extern "C" int mpcx_sk_run(mpcx_sk* e, int64_t ncoll, const double* draws, int64
     // device draws: the far particles stream and bin beside the near engine
     // (host draws: the shift is read at the draw cursor the near engine moves)
     const bool ov = e->overlap && P.rng_mode == 1 && !sort_due;
-    auto near = [&](int mode, int nmot) {   // the near engine's launch of nmot motions
+    // The near engine needs a CU's LDS nearly whole: its dispatch must find one
+    // that the far stream has not filled, so the fork comes after sk_near_split,
+    // with nothing left between it and the near engine.
+    auto near = [&](int mode, int nmot, bool fork) -> hipError_t {   // the near engine's launch of nmot motions
       if (P.rng_mode != 0) hipLaunchKernelGGL(sk_near_split, dim3(64), dim3(256), 0, st, P, D, nmot);
+      const hipError_t r = fork ? hipEventRecord(e->fork, st) : hipSuccess;
       hipLaunchKernelGGL(sk_near_engine, dim3(1), dim3(SK_T), 0, st, P, D, mode);
+      return r;
     };
-    if (ov) SKCHK(hipEventRecord(e->fork, st));
     SKCHK(tmark(0, 0));
-    if (sort_due) near(SM_STOP, P.S - 1);
-    else near(0, P.S);
+    SKCHK(sort_due ? near(SM_STOP, P.S - 1, false) : near(0, P.S, ov));
     SKCHK(tmark(0, 1));
-    if (ov) {   // enqueued after the near engine, so that it is dispatched first
+    if (ov) {
       SKCHK(hipStreamWaitEvent(e->st2, e->fork, 0));
       if (timed) {
         e->tev_on[(size_t)slot * mpcx_sk::NKT + 1] = 1;
@@ -1751,7 +1754,7 @@ extern "C" int mpcx_sk_run(mpcx_sk* e, int64_t ncoll, const double* draws, int64
       hipLaunchKernelGGL(sk_bulk, dim3(gN), dim3(256), 0, st, P, D, P.S - 1, 0, 0);
       sk_sort(e);
       sk_near_list(e);
-      near(SM_RESUME, 1);
+      SKCHK(near(SM_RESUME, 1, false));
       hipLaunchKernelGGL(sk_bulk, dim3(gN), dim3(256), 0, st, P, D, 1, 1, 0);
     } else {
       SKCHK(tmark(1, 0));
