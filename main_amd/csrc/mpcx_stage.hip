@@ -257,8 +257,11 @@ bool pageable(const void* p) {
 }
 
 int copy(const std::vector<HostCopy>& v, bool out, hipStream_t st) {
+  size_t all = 0, total = 0;
+  for (const HostCopy& c : v)
+    if (c.host) all += c.bytes;
+  if (all < MIN_STAGED) return plain(v, out, st);
   std::vector<HostCopy> ring, rest;
-  size_t total = 0;
   for (const HostCopy& c : v) {
     if (!c.host || !c.bytes) continue;
     const bool r = c.widen || pageable(c.host);   // (widening is host work whatever the memory)
