@@ -101,13 +101,9 @@ struct SkD {
 
 __device__ __forceinline__ int species(int f) { return f == 0 ? 0 : f == 1 ? 1 : f == 3 ? 2 : -1; }
 __device__ __forceinline__ bool active(int f) { return f == 0 || f == 1 || f == 3; }
-// x - L*floor(x/L) without the division for -L <= x < 2L: a correctly rounded
-// x/L lies in [-1,0), [0,1) or [1,2) exactly when x does, so the floor follows
-// by comparison and the subtraction is the same operation
-__device__ __forceinline__ double wrap(double x, double L) {
-  if (__builtin_expect(x < -L || x >= 2.0 * L, 0)) return x - L * floor(x / L);
-  return x < 0.0 ? x + L : (x >= L ? x - L : x);
-}
+// (by comparisons instead of the division, which is bitwise the same for
+// -L <= x < 2L, a near engine's launch took 3 to 4 % longer in both its forms)
+__device__ __forceinline__ double wrap(double x, double L) { return x - L * floor(x / L); }
 
 // INT(FLOOR(X)+Box(1)*FLOOR(Y)+Box(1)*Box(2)*FLOOR(Z)+1) - 1
 __device__ __forceinline__ long long sk_cell0(const SkP& P, double x, double y, double z) {
