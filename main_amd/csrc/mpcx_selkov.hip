@@ -433,13 +433,24 @@ __device__ __attribute__((noinline)) void sk_step(bool last, bool census) {
   __syncthreads();
 }
 
-// gather the near set from the particle arrays, and scatter it back
-__device__ __forceinline__ void sk_gather(const SkD& D, int nn) {
+__device__ __forceinline__ SkSlot sk_particle(const SkD& D, int p) {
+  SkSlot s;
+  s.x = D.x[p]; s.y = D.y[p]; s.z = D.z[p]; s.vx = D.vx[p]; s.vy = D.vy[p]; s.vz = D.vz[p];
+  s.fx = D.fx[p]; s.fy = D.fy[p]; s.fz = D.fz[p]; s.flag = D.flag[p];
+  return s;
+}
+// gather the near set from the particle arrays, and scatter it back; after
+// sk_near_split (split) the slots of the particles that matter hold their state
+// already, side by side where the particle arrays are scattered
+enum : unsigned char { NF_MATTER = 0x40 };
+__device__ __forceinline__ void sk_gather(const SkD& D, int nn, bool split) {
   for (int q = threadIdx.x; q < nn; q += SK_T) {
-    const int p = D.near_list[q];
     SkSlot s;
-    s.x = D.x[p]; s.y = D.y[p]; s.z = D.z[p]; s.vx = D.vx[p]; s.vy = D.vy[p]; s.vz = D.vz[p];
-    s.fx = D.fx[p]; s.fy = D.fy[p]; s.fz = D.fz[p]; s.flag = D.flag[p];
+    if (split && (D.ns_cflag[q] & NF_MATTER))
+      s = SkSlot{D.ns_x[q], D.ns_y[q], D.ns_z[q], D.ns_vx[q], D.ns_vy[q], D.ns_vz[q],
+                 D.ns_fx[q], D.ns_fy[q], D.ns_fz[q], D.ns_flag[q]};
+    else
+      s = sk_particle(D, D.near_list[q]);
     slot_store(D, q, s);
     D.ns_cflag[q] = (unsigned char)s.flag;
   }
@@ -550,12 +561,6 @@ __device__ __forceinline__ void sk_fly(const SkP& P, SkSlot& s, int moves) {
     s.z = wrap(s.z + dz, P.box[2]);
   }
 }
-__device__ __forceinline__ SkSlot sk_particle(const SkD& D, int p) {
-  SkSlot s;
-  s.x = D.x[p]; s.y = D.y[p]; s.z = D.z[p]; s.vx = D.vx[p]; s.vy = D.vy[p]; s.vz = D.vz[p];
-  s.fx = D.fx[p]; s.fy = D.fy[p]; s.fz = D.fz[p]; s.flag = D.flag[p];
-  return s;
-}
 __device__ __forceinline__ double sk_min_image2(const SkP& P, double x, double y, double z, int sph, double& d1, double& d2,
                                                 double& d3) {
   d1 = x - g_sk.sd[SX][sph];
@@ -574,7 +579,6 @@ __device__ __forceinline__ double sk_min_image2(const SkP& P, double x, double y
 // set lies scattered over the particle arrays (they are re-sorted every 10,000
 // steps), so its gather is the work of the whole chip: by the near engine's one
 // CU it took 0.2 ms, more than the MD steps.
-enum : unsigned char { NF_MATTER = 0x40 };
 __global__ __launch_bounds__(256) void sk_near_split(SkP P, SkD D, int nmot) {
   __shared__ double sd[3][2];
   if (threadIdx.x < 6) sd[threadIdx.x >> 1][threadIdx.x & 1] = D.dim[(SX + (threadIdx.x >> 1)) * 2 + (threadIdx.x & 1)];
@@ -840,7 +844,7 @@ __global__ __launch_bounds__(SK_T) void sk_near_engine(SkP P, SkD D, int mode) {
   int t = t0;
   const bool fast = P.rng_mode != 0 && t0 <= t1 && sk_steps(P, D, nn, t0, t1, t);
   if (!fast) {
-    sk_gather(D, nn);
+    sk_gather(D, nn, P.rng_mode != 0);
     __threadfence_block();
     __syncthreads();
     // motion of the launch's first step, solvent and dimer
