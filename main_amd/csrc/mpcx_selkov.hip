@@ -818,6 +818,9 @@ __device__ __forceinline__ bool sk_steps(const SkP& P, const SkD& D, int nn, int
 // mode 0: steps 1..S of an interval (motion of step 1 first);
 // SM_STOP: steps 1..S-1, without the motion of step S (a sort comes first);
 // SM_RESUME: the motion and the step S.
+// STEPS (device draws): sk_steps where it can; else the general form alone, as
+// the parity stream needs it (compiled together its launches took 1 % longer).
+template <bool STEPS>
 __global__ __launch_bounds__(SK_T) void sk_near_engine(SkP P, SkD D, int mode) {
   const int tid = threadIdx.x;
   SkScalars* sc = D.sc;
@@ -842,9 +845,10 @@ __global__ __launch_bounds__(SK_T) void sk_near_engine(SkP P, SkD D, int mode) {
   const int t0 = (mode & SM_RESUME) ? P.S : 1;
   const int t1 = (mode & SM_STOP) ? P.S - 1 : P.S;
   int t = t0;
-  const bool fast = P.rng_mode != 0 && t0 <= t1 && sk_steps(P, D, nn, t0, t1, t);
+  bool fast = false;
+  if constexpr (STEPS) fast = t0 <= t1 && sk_steps(P, D, nn, t0, t1, t);
   if (!fast) {
-    sk_gather(D, nn, P.rng_mode != 0);
+    sk_gather(D, nn, STEPS);
     __threadfence_block();
     __syncthreads();
     // motion of the launch's first step, solvent and dimer
@@ -1729,9 +1733,11 @@ extern "C" int mpcx_sk_run(mpcx_sk* e, int64_t ncoll, const double* draws, int64
     // that the far stream has not filled, so the fork comes after sk_near_split,
     // with nothing left between it and the near engine.
     auto near = [&](int mode, int nmot, bool fork) -> hipError_t {   // the near engine's launch of nmot motions
-      if (P.rng_mode != 0) hipLaunchKernelGGL(sk_near_split, dim3(64), dim3(256), 0, st, P, D, nmot);
+      const bool steps = P.rng_mode != 0;
+      if (steps) hipLaunchKernelGGL(sk_near_split, dim3(64), dim3(256), 0, st, P, D, nmot);
       const hipError_t r = fork ? hipEventRecord(e->fork, st) : hipSuccess;
-      hipLaunchKernelGGL(sk_near_engine, dim3(1), dim3(SK_T), 0, st, P, D, mode);
+      if (steps) hipLaunchKernelGGL(sk_near_engine<true>, dim3(1), dim3(SK_T), 0, st, P, D, mode);
+      else hipLaunchKernelGGL(sk_near_engine<false>, dim3(1), dim3(SK_T), 0, st, P, D, mode);
       return r;
     };
     SKCHK(tmark(0, 0));
