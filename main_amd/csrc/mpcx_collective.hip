@@ -2130,15 +2130,6 @@ __device__ __forceinline__ int block_groups(const CoP& P, const CoD& D, GroupTab
   return ok ? G.rb[rs] + local : 0;
 }
 
-// Binning of one particle per lane; every thread of the block calls it
-// together (`valid` false for idle lanes).  The shifted cell, counted by tour
-// position with the particle's rank in it; the distance to the nearest sphere
-// of `sph` beyond its list radius (selection of the next interval's near set);
-// the census of distribute_mod.f95:95-183: outside particles keyed by index,
-// inside ones after all outside ones, inside ones within a cutoff skipped.
-// slab 0: cell and rank for co_scatter; 1: the particle's slot in its cell's
-// slab written directly; 2: the same, and the cell must be listed late (the
-// particle was binned after the first collision pass).
 // Distance beyond the nearest list radius; 8 or more beyond every radius gives
 // 1e30 (the cap, 255 at 7.97) without a square root.
 __device__ __forceinline__ double list_distance(const CoP& P, double x, double y, double z, const double (*sph)[MAXSG]) {
@@ -2211,6 +2202,15 @@ __device__ __forceinline__ double list_distance_culled(const CoP& P, bool valid,
   return dmin;
 }
 
+// Binning of one particle per lane; every thread of the block calls it
+// together (`valid` false for idle lanes).  The shifted cell, counted by tour
+// position with the particle's rank in it; the distance to the nearest sphere
+// of `sph` beyond its list radius (selection of the next interval's near set);
+// the census of distribute_mod.f95:95-183: outside particles keyed by index,
+// inside ones after all outside ones, inside ones within a cutoff skipped.
+// slab 0: cell and rank for co_scatter; 1: the particle's slot in its cell's
+// slab written directly; 2: the same, and the cell must be listed late (the
+// particle was binned after the first collision pass).
 // CULL: systems of any number of dimers (else the few of a one-workgroup near engine)
 template <bool CULL>
 __device__ __forceinline__ void bin_particle(const CoP& P, const CoD& D, int i, bool valid, bool near,
