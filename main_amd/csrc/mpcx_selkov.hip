@@ -211,7 +211,7 @@ struct SkShared {
   int wsum[SK_W + 1];
   long long cursor, cstep;
   int nn;
-  double x0[3][2];   // spheres at the interval start (guard check)
+  double x0[3][2];   // spheres at the interval start (guard check of sk_dimer_step)
   SkP P;
   SkD D;
 };
@@ -287,6 +287,8 @@ __device__ __forceinline__ void sk_wave_scan() {
 
 __device__ __attribute__((noinline)) void sk_begin_motion() {
   // thread 0: the dimer part of Motion_SelkovDimer for the next step, and the guard check
+  // (the spheres' starts from memory: they arrive beside the motion; read from
+  // LDS at its end they made a launch 1 % longer)
   const SkP& P = g_sk.P;
   const SkD& D = g_sk.D;
   Dim2 d;
@@ -298,9 +300,9 @@ __device__ __attribute__((noinline)) void sk_begin_motion() {
   g_sk.bond[0] = d.bond[0]; g_sk.bond[1] = d.bond[1]; g_sk.bond[2] = d.bond[2];
 #pragma unroll
   for (int s = 0; s < 2; s++) {
-    double a = pbc_h(d.v[SX][s] - g_sk.x0[0][s], P.hbox[0], P.box[0]);
-    double b = pbc_h(d.v[SY][s] - g_sk.x0[1][s], P.hbox[1], P.box[1]);
-    double c = pbc_h(d.v[SZ][s] - g_sk.x0[2][s], P.hbox[2], P.box[2]);
+    double a = pbc_h(d.v[SX][s] - D.sc->x0[s], P.hbox[0], P.box[0]);
+    double b = pbc_h(d.v[SY][s] - D.sc->y0[s], P.hbox[1], P.box[1]);
+    double c = pbc_h(d.v[SZ][s] - D.sc->z0[s], P.hbox[2], P.box[2]);
     if (a * a + b * b + c * c > P.guard * P.guard) raise_error(&D.sc->err, ERR_NEAR_GUARD);
   }
 }
