@@ -5966,11 +5966,12 @@ static void sb_launch_bulk(mpcx_cob* b, bool all, hipStream_t s, int bin) {
 // CUs free) the far particles' flight and binning (st2) run beside the near
 // engine (st); the near set is binned on st when it is done; every cell is
 // collided and every particle rotated once both are.  A batch runs them in
-// order: its near engines hold a CU each (LDS and VGPRs), so a far flight
-// launched beside them only waits for CUs, in dispatch order, and started
-// beside them or beside the near sets' binning it measured 3.78 and 3.81 ms
-// per interval of the 256-replica ensemble against 3.77 in order.  A re-sort interval
-// stops the near engines before the last step's list rebuild (the far flight
+// order: its near engines hold a CU each (LDS and VGPRs), so with a replica for
+// every CU a far flight launched beside them only waits for CUs, in dispatch
+// order, and started beside them or beside the near sets' binning it measured
+// 3.78 and 3.81 ms per interval of the 256-replica ensemble against 3.77 in
+// order.  (Not measured for fewer replicas, whose near engines leave the other
+// CUs idle.)  A re-sort interval stops the near engines before the last step's list rebuild (the far flight
 // is not binned), re-sorts, lets them resume, then bins every particle.
 // slot >= 0: the interval's kernels are timed (events into that slot).
 static int sb_interval(mpcx_cob* b, bool sort_due, long long slot) {

@@ -554,11 +554,17 @@ __device__ __forceinline__ void sk_reduce(const double (&a)[7], int wv, int lane
 // go through LDS to the lane the general form sums them in, in its order
 // (entries ascending), so the sums are its sums bitwise.  In the general form
 // every step moved the whole set through LDS and L2 and one thread took the
-// dimer's step: 37 us a step at 50^3, 0.74 ms a launch.
+// dimer's step: 37 us a step at 50^3, 0.74 ms a launch (0.13 alone and 0.15
+// beside sk_bulk so).
 //
 // Device draws only: the parity stream's draws follow the order of the whole
 // set.  Returns false, with nothing done, when more than SK_A particles
-// matter; else `t_next` is the step after the last one done (before t1 + 1: the
+// matter, as many as the threads' registers hold; the general form then takes
+// the launch, at its speed before this form was there.  The line lies at
+// radii of some 3 and 5 at 10 a cell, T = 1 and a guard of 1 (40^3: 1,140 that
+// matter with radii 2 and 4, 0.30 ms an interval; 2,082 with 3 and 5, 1.18 ms;
+// 3,373 with 4 and 6, 1.66), below radii 2 and 4 at 20 a cell (2,244, 1.48 ms)
+// or T = 10 (2,547, 0.99 ms).  Else `t_next` is the step after the last one done (before t1 + 1: the
 // spheres moved too far, the slots hold every particle at that step's start).
 constexpr double SK_QUIET = 0.1;   // of the guard: a sphere moves some 0.003 a launch at 50^3, a wider shell holds more particles
 __device__ __forceinline__ void sk_fly(const SkP& P, SkSlot& s, int moves) {
